@@ -347,6 +347,51 @@ def test_graph_mode_matches_eager(gpu, cfg):
     assert ar_e == ar_g
 
 
+def test_capture_next_to_collectable_engine(gpu):
+    """An engine with captured graphs that only a cyclic collection can free
+    (it sits in a reference cycle) leaves captures of another engine alone:
+    with the collector due at every allocation, the graph run commits the
+    eager run's tokens, and the old engine is gone afterwards."""
+    import gc
+    import weakref
+
+    cfg = TINY
+    w = M.init_weights(cfg, 2)
+    ids = _prompt(40, 11).to(gpu)
+    pol = SsdPolicy(cfg.T_total, 2)
+    mk = lambda graphs: LoopedBlocks(LoopedModel(cfg, w, gpu, max_seq_len=80, use_graphs=graphs))  # noqa: E731
+    eager, _ = generate_wavefront_dynamic(mk(False), ids, 8, pol)
+    old = mk(True)
+    assert generate_wavefront_dynamic(old, ids, 8, pol)[0] == eager
+    old.model.me = old.model
+    gone = weakref.ref(old.model)
+    new = mk(True)
+    torch.cuda.synchronize()
+    thresholds = gc.get_threshold()
+    collect, gc_during = gc.isenabled, []
+    launch = new.model._launch_plans
+
+    def noting(*a, **kw):
+        if torch.cuda.is_current_stream_capturing():
+            gc_during.append(collect())
+        return launch(*a, **kw)
+
+    new.model._launch_plans = noting
+    gc.disable()
+    del old
+    try:
+        gc.set_threshold(1, 1, 1)
+        gc.enable()
+        print("[capture next to a collectable engine]", flush=True)
+        got, _ = generate_wavefront_dynamic(new, ids, 8, pol)
+    finally:
+        gc.set_threshold(*thresholds)
+        new.model.__dict__.pop("_launch_plans", None)
+    assert gc_during and not any(gc_during) and gc.isenabled()
+    gc.collect()
+    assert gone() is None and got == eager
+
+
 def test_graph_mode_batch_emulated(gpu):
     cfg = TINY
     w = M.init_weights(cfg, 0)

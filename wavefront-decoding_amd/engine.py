@@ -39,6 +39,10 @@ reuses its position's row.
 """
 from __future__ import annotations
 
+import contextlib
+import gc
+import threading
+
 import numpy as np
 import torch
 
@@ -82,6 +86,28 @@ class _Staging:
             dt = {np.dtype(np.int32): torch.int32, np.dtype(np.int64): torch.int64}[a.dtype]
             out.append(self.dev[j][o: o + a.nbytes].view(dt).view(a.shape))
         return out
+
+
+_no_gc_lock = threading.RLock()
+
+
+@contextlib.contextmanager
+def _no_gc():
+    """Python's cyclic collector held off while a stream is being captured. An
+    engine that sits in a reference cycle is freed by whichever allocation
+    happens to trigger a collection; inside a capture its destructors would
+    synchronize, destroy graphs and events and return pinned buffers whose
+    stream use the allocator records -- calls a capturing process may not
+    make, and an error raised in a destructor ends the process. Captures of
+    several threads take turns."""
+    with _no_gc_lock:
+        was = gc.isenabled()
+        gc.disable()
+        try:
+            yield
+        finally:
+            if was:
+                gc.enable()
 
 
 class _Captured:
@@ -581,7 +607,7 @@ class LoopedModel:
         self._launch_plans(cache, plans, g.d32, g.d64, cache.S)                   # warm-up, then capture
         torch.cuda.synchronize()
         g.graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(g.graph):
+        with _no_gc(), torch.cuda.graph(g.graph):
             self._launch_plans(cache, plans, g.d32, g.d64, cache.S)
         torch.cuda.synchronize()
         g.exec = g.graph.raw_cuda_graph_exec()
