@@ -41,10 +41,11 @@ enum { WFD_EPI_PLAIN = 0, WFD_EPI_SWIGLU = 1 };
 
 /* Message for the last failing call on this thread. */
 const char* wfd_last_error(void);
-/* Bumped whenever an entry point's signature changes or one is added (5: wfd_argmax's
+/* Bumped whenever an entry point's signature changes (5: wfd_argmax's
    accept flags, wfd_attn_varlen_rows; 6: wfd_linear_argmax, wfd_argmax_groups;
    7: folded norm pairs -- wfd_linear_prep, wfd_norm_prep, the row-scale argument of
-   wfd_linear, wfd_linear_qkv_rope_append and wfd_linear_argmax). */
+   wfd_linear, wfd_linear_qkv_rope_append and wfd_linear_argmax; wfd_attn_varlen
+   joined at 7, which changed no signature). */
 int wfd_abi_version(void);
 
 /*
@@ -167,6 +168,27 @@ int wfd_attn_decode_noalloc(const void* q, const void* k_cache, const void* v_ca
  */
 int wfd_attn_varlen_rows(const int32_t* cu_q, const int32_t* cu_k, int nseg, int total_q, int causal,
                          int64_t* kv_row_base, int32_t* kv_len, wfd_stream_t stream);
+
+/*
+ * Packed varlen attention in one call (bf16; Dh 64 or 128; H / Hkv in {1, 2,
+ * 4}; scale > 0): out row r of segment s (rows [cu_q[s], cu_q[s+1]) of q
+ * (total_q, H, Dh)) attends keys of [cu_k[s], cu_k[s+1]) of the token-major k /
+ * v (total_k, Hkv, Dh) -- the whole segment, or bottom-right causal, exactly
+ * the keys wfd_attn_varlen_rows gives the row; a row without keys, or outside
+ * every segment, is zero. The call for segments of several rows: up to 32 /
+ * (H / Hkv) rows of a segment read each key together on MFMA, where
+ * wfd_attn_decode reads a row's keys for that row alone. fp32 softmax and
+ * sums; the probabilities enter the second product as two bf16 terms (16
+ * significant bits). A row's bits depend on its own keys only. max_k >= every
+ * segment's key count sizes the grid. workspace >=
+ * wfd_attn_varlen_workspace_bytes(...), 16-byte aligned; q, k, v and out too.
+ * Replaces: fa4_attention.attn_varlen / _attn_varlen_torch
+ *   (src/decoding/fa4_attention.py:301-317,348-366).
+ */
+size_t wfd_attn_varlen_workspace_bytes(int nseg, int total_q, int H, int Hkv, int Dh, int max_k);
+int wfd_attn_varlen(const void* q, const void* k, const void* v, const int32_t* cu_q, const int32_t* cu_k, void* out,
+                    int nseg, int total_q, int H, int Hkv, int Dh, int dtype, float scale, int max_k, int causal,
+                    void* workspace, size_t ws_bytes, wfd_stream_t stream);
 
 /*
  * Causal prefill attention on MFMA (bf16; Dh 64 or 128; any H / Hkv).

@@ -62,6 +62,72 @@ def test_attn_varlen_matches_oracle(gpu, dtype, causal, H, Hkv, Dh):
         assert torch.count_nonzero(out[cu_q[2]: cu_q[2] + 2].float()) == 0
 
 
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("H,Hkv,Dh", [(4, 4, 128), (8, 2, 128), (4, 2, 64), (2, 2, 64)])
+def test_attn_varlen_shared_rows(gpu, causal, H, Hkv, Dh):
+    """The kernel that reads a key once for the rows of a segment, at the edges
+    of its row tiles (32 / G rows), key tiles (32) and splits (1024), with rows
+    outside every segment, an empty segment, segments with fewer keys than rows
+    and none, and more segments than its table workgroup has threads. Error
+    against float64 relative to the result's norm: at most the bf16 output
+    rounding (2^-9) plus that of the probabilities' two bf16 terms (2^-17),
+    three times over for rows whose values cancel. A row alone in its segment
+    (bottom-right causal: its last row) has the same bits as in the full one."""
+    T = 32 // (H // Hkv)
+    seg = [(T, 31), (1, 32), (T + 1, 33), (0, 5), (2 * T - 1, 1024), (3, 1025), (2, 2100), (5, 2), (4, 0), (1, 1)]
+    seg += [(1 + i % 2, 1 + i % 40) for i in range(300)]
+    lead, tail = 3, 2
+    cu_q = lead + np.concatenate([[0], np.cumsum([a for a, _ in seg])]).astype(np.int32)
+    cu_k = np.concatenate([[0], np.cumsum([b for _, b in seg])]).astype(np.int32)
+    n = int(cu_q[-1]) + tail
+    g = torch.Generator().manual_seed(H + Dh + causal)
+    mk = lambda r, h: torch.randn(r, h, Dh, generator=g).to(torch.bfloat16)  # noqa: E731
+    q, k, v = mk(n, H), mk(int(cu_k[-1]), Hkv), mk(int(cu_k[-1]), Hkv)
+    print(f"[attn_varlen shared rows] causal={causal} H={H} Hkv={Hkv} Dh={Dh}", flush=True)
+    dev = [t.to(gpu) for t in (q, k, v)]
+    cq, ck = torch.from_numpy(cu_q).to(gpu), torch.from_numpy(cu_k).to(gpu)
+    out = A.attn_varlen(*dev, cq, ck, max(a for a, _ in seg), max(b for _, b in seg), causal=causal)
+    ref = np.zeros((n, H, Dh))
+    ref[lead: int(cu_q[-1])] = _varlen_ref(q[lead:], k, v, cu_q - lead, cu_k, causal)[: int(cu_q[-1]) - lead]
+    got = _np(out)
+    assert np.linalg.norm(got - ref) <= 3 * 2.0 ** -9 * np.linalg.norm(ref)
+    assert rel_err(got, ref) <= TOL[torch.bfloat16]
+    assert not got[:lead].any() and not got[n - tail:].any()  # outside every segment
+    # the last row of each of the first segments, among one-row segments and a two-row one
+    last = [i for i, (a, _) in enumerate(seg[:10]) if a > 0]
+    rows = torch.tensor([int(cu_q[i + 1]) - 1 for i in last], device=gpu)
+    qs = torch.cat([dev[0][rows], dev[0][:2]])
+    ks = torch.cat([dev[1][cu_k[i]: cu_k[i + 1]] for i in last] + [dev[1][:7]])
+    vs = torch.cat([dev[2][cu_k[i]: cu_k[i + 1]] for i in last] + [dev[2][:7]])
+    kl = [seg[i][1] for i in last] + [7]
+    off = lambda x: torch.tensor(np.concatenate([[0], np.cumsum(x)]), dtype=torch.int32, device=gpu)  # noqa: E731
+    alone = A.attn_varlen(qs, ks, vs, off([1] * len(last) + [2]), off(kl), 2, max(kl), causal=causal)
+    assert torch.equal(alone[: len(last)], out[rows])
+
+
+def test_attn_varlen_shared_rows_special_values(gpu):
+    """Infinities and NaN stay with the rows that attend them: a causal segment
+    whose last keys' V hold them leaves the rows before those keys finite (and,
+    before the 32-key tile that holds them, bit for bit the same), and the rows
+    that attend an infinity get it."""
+    g = torch.Generator().manual_seed(3)
+    n, H, Dh = 60, 2, 128
+    q, k, v = (torch.randn(n, H, Dh, generator=g).to(torch.bfloat16).to(gpu) for _ in range(3))
+    cu = torch.tensor([0, n], dtype=torch.int32, device=gpu)
+    plain = A.attn_varlen(q, k, v, cu, cu, n, n, causal=True)
+    v[40, 0, 5] = float("inf")
+    v[50, 1, 7] = float("nan")
+    got = A.attn_varlen(q, k, v, cu, cu, n, n, causal=True)
+    assert torch.equal(got[:32], plain[:32])
+    assert torch.isinf(got[40:, 0, 5]).all() and torch.isnan(got[50:, 1, 7]).all()
+    clean = torch.ones_like(got, dtype=torch.bool)
+    clean[40:, 0, 5] = clean[50:, 1, 7] = False
+    assert torch.isfinite(got[clean].float()).all()
+    # the tile that holds them was summed key by key in fp32: the other values agree to bf16 rounding
+    d = (got.float() - plain.float())[clean].norm() / plain.float()[clean].norm()
+    assert d <= 2.0 ** -8
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_attn_varlen_q1_padded_matches_oracle(gpu, dtype):
     lens = [1, 64, 300, 1025, 7]

@@ -9,12 +9,17 @@ runs a HIP kernel of libwfd.so on torch's current stream:
 
   attn_dense      bf16 causal with Tq <= Tk (a prompt, bottom-right aligned):
                   the MFMA prefill kernel (wfd_attn_prefill), one segment per
-                  batch row; otherwise the decode kernel (wfd_attn_decode)
-                  with one (row base, key count) entry per query row
+                  batch row; any other bf16 call with Tq > 1: the varlen kernel
+                  (wfd_attn_varlen), one segment per batch row; otherwise the
+                  decode kernel (wfd_attn_decode) with one (row base, key
+                  count) entry per query row
   attn_cutoff_multi  the decode kernel with key count = qpos + 1
-  attn_varlen     the decode kernel over the packed K / V (token-major), its
-                  row tables expanded from cu_q / cu_k on the device
-                  (wfd_attn_varlen_rows), so nothing is read back to the host
+  attn_varlen     bf16 with more rows than segments: the varlen kernel, whose
+                  workgroups read a key once for up to 32 / (H / Hkv) rows of
+                  its segment; otherwise (a row per segment, fp32) the decode
+                  kernel over the packed K / V (token-major), its row tables
+                  expanded from cu_q / cu_k on the device
+                  (wfd_attn_varlen_rows). Nothing is read back to the host
   attn_varlen_q1_padded  attn_varlen with one query row per segment (the
                   reference pads each to two causal rows to steer FA2's tile
                   choice; the decode kernel has no such template switch, and
@@ -99,6 +104,22 @@ def _prefill_segments(B: int, Tq: int, Tk: int, device):
     return _cached(("prefill", B, Tq, Tk, str(device)), build)
 
 
+def _shared_rows(q: torch.Tensor, k: torch.Tensor) -> bool:
+    """Whether the kernel that reads a key once for all rows of a segment
+    (wfd_attn_varlen) takes these heads: bf16, Dh 64 / 128, 1, 2 or 4 query
+    heads per kv head."""
+    H, Dh, Hkv = q.shape[-2], q.shape[-1], k.shape[-2]
+    return q.dtype == k.dtype == torch.bfloat16 and Dh in (64, 128) and Hkv > 0 and H in (Hkv, 2 * Hkv, 4 * Hkv)
+
+
+def _dense_offsets(B: int, Tq: int, Tk: int, device):
+    def build():
+        s = torch.arange(B + 1, dtype=torch.int32)
+        return (s * Tq).to(device), (s * Tk).to(device)
+
+    return _cached(("dense_cu", B, Tq, Tk, str(device)), build)
+
+
 def attn_dense(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, causal: bool) -> torch.Tensor:
     """q (B, Tq, H, Dh), k / v (B, Tk, Hkv, Dh) -> (B, Tq, H, Dh). causal is
     bottom-right aligned (query i attends keys <= i + Tk - Tq); a lone query
@@ -113,6 +134,9 @@ def attn_dense(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, causal: boo
     if causal and Tq > 1 and Tq <= Tk and q.dtype == torch.bfloat16 and Dh in (64, 128):
         rb, qs, p0 = _prefill_segments(B, Tq, Tk, q.device)
         out = ops.attn_prefill(qf, kf, vf, rb, qs, p0, max_seg_len=Tq, scale=_scale(Dh))
+    elif Tq > 1 and _shared_rows(q, k):
+        cq, ck = _dense_offsets(B, Tq, Tk, q.device)
+        out = ops.attn_varlen(qf, kf, vf, cq, ck, max_k=max(Tk, 1), causal=causal, scale=_scale(Dh))
     else:
         rb, kl = _dense_rows(B, Tq, Tk, causal and Tq > 1, q.device)
         out = ops.attn_decode(qf, kf, vf, rb, kl, kv_len_max=max(Tk, 1), scale=_scale(Dh))
@@ -151,6 +175,9 @@ def attn_varlen(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu_q: torch.T
         raise _lib.WfdError("attn_varlen: q (total_q, H, Dh), k / v (total_k, Hkv, Dh)")
     cq = cu_q.to(device=q.device, dtype=torch.int32).contiguous()
     ck = cu_k.to(device=q.device, dtype=torch.int32).contiguous()
+    if total_q >= cq.numel() and _shared_rows(q, k):  # some segment brings more than one row
+        return ops.attn_varlen(q.contiguous(), k.contiguous(), v.contiguous(), cq, ck, max_k=max(int(max_k), 1),
+                               causal=causal, scale=_scale(Dh))
     rb, kl = ops.attn_varlen_rows(cq, ck, total_q, causal=causal)
     return ops.attn_decode(q.contiguous(), k.contiguous(), v.contiguous(), rb, kl, kv_len_max=max(int(max_k), 1),
                            scale=_scale(Dh))

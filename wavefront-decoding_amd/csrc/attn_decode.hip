@@ -40,13 +40,9 @@
 // the B=32 decode 13 % faster; uniform long prefixes lose ~2-3 %.
 #include <mutex>
 
-#include "wfd_common.h"
+#include "attn_combine.h"
 
 namespace wfd {
-
-constexpr int kAttnSplit = 1024;  // keys per workgroup
-
-__device__ __forceinline__ float attn_finish(float O, float L) { return L > 0.f ? O / L : 0.f; }
 
 // One workgroup = (split, kv head g, group of QG query rows that share a slot).
 // MFMA row m = j * G + r carries query row j of the group at query head
@@ -373,93 +369,12 @@ __global__ __launch_bounds__(64 * NW) void attn_split_kernel(const T* __restrict
   }
 }
 
-// Merge of a row's split partials, in split order: M = max m_s, then
-// L = sum l_s * 2^(m_s - M) and O = sum o_s * 2^(m_s - M), one fma per split.
-// The partials are read in batches of kCombineBatch independent loads, so a
-// row of many splits waits on memory twice per batch, not twice per split.
-constexpr int kCombineBatch = 8;
-
-template <typename T, int DH>
-__global__ __launch_bounds__(DH) void attn_combine_kernel(const float* __restrict__ part_o,
-                                                          const float* __restrict__ part_ml,
-                                                          const int32_t* __restrict__ kv_len, T* __restrict__ out,
-                                                          int H, int max_splits) {
-  constexpr int B = kCombineBatch;
-  const int h = blockIdx.x;
-  const int i = blockIdx.y;
-  const int d = threadIdx.x;
-  const int len = kv_len[i];
-  int ns = len > 0 ? (len + kAttnSplit - 1) / kAttnSplit : 0;
-  ns = min(ns, max_splits);
-  if (ns <= 1) return;  // finished by its split workgroup
-  const int64_t base = ((int64_t)i * H + h) * max_splits;
-  float M = -INFINITY;
-  for (int s0 = 0; s0 < ns; s0 += B) {
-    float mv[B];
-#pragma unroll
-    for (int b = 0; b < B; ++b) mv[b] = s0 + b < ns ? part_ml[(base + s0 + b) * 2] : -INFINITY;
-#pragma unroll
-    for (int b = 0; b < B; ++b) M = fmaxf(M, mv[b]);
-  }
-  float O = 0.f, L = 0.f;
-  for (int s0 = 0; s0 < ns; s0 += B) {
-    float mv[B], lv[B], ov[B];
-#pragma unroll
-    for (int b = 0; b < B; ++b) {
-      const bool ok = s0 + b < ns;
-      mv[b] = ok ? part_ml[(base + s0 + b) * 2] : -INFINITY;
-      lv[b] = ok ? part_ml[(base + s0 + b) * 2 + 1] : 0.f;
-      ov[b] = ok ? part_o[(base + s0 + b) * DH + d] : 0.f;
-    }
-#pragma unroll
-    for (int b = 0; b < B; ++b) {
-      if (s0 + b < ns) {
-        const float f = (mv[b] == -INFINITY) ? 0.f : exp2f(mv[b] - M);
-        L = fmaf(lv[b], f, L);
-        O = fmaf(ov[b], f, O);
-      }
-    }
-  }
-  Elem<T>::store(out + ((int64_t)i * H + h) * DH + d, attn_finish(O, L));
-}
-
-// Per-row tables of a packed varlen call (the FA varlen convention): query
-// row r of segment s (rows [cu_q[s], cu_q[s+1]), keys [cu_k[s], cu_k[s+1]) of
-// a token-major K / V) reads keys from row cu_k[s]; non-causal it reads the
-// whole segment, causal (bottom-right) keys [0, k_len - q_len + r - cu_q[s]].
-// Rows at or past cu_q[nseg] get no keys. One thread per row, a binary search
-// over cu_q: the tables never leave the device.
+// Row tables of a packed varlen call, one thread per row (varlen_row).
 __global__ void varlen_rows_kernel(const int32_t* __restrict__ cu_q, const int32_t* __restrict__ cu_k, int nseg,
                                    int total_q, int causal, int64_t* __restrict__ row_base,
                                    int32_t* __restrict__ kv_len) {
   const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= total_q) return;
-  int lo = 0, hi = nseg;  // find the last s with cu_q[s] <= r
-  if (nseg <= 0 || r >= cu_q[nseg] || r < cu_q[0]) {
-    row_base[r] = 0;
-    kv_len[r] = 0;
-    return;
-  }
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (cu_q[mid] <= r)
-      lo = mid;
-    else
-      hi = mid;
-  }
-  const int qs = cu_q[lo], ql = cu_q[lo + 1] - qs;
-  const int ks = cu_k[lo], kl = cu_k[lo + 1] - ks;
-  row_base[r] = ks;
-  kv_len[r] = causal ? max(kl - ql + (r - qs) + 1, 0) : kl;
-}
-
-static int max_splits_for(int kv_len_max) { return kv_len_max <= 0 ? 1 : (kv_len_max + kAttnSplit - 1) / kAttnSplit; }
-
-static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
-
-static size_t attn_ws_bytes(int n, int H, int Dh, int kv_len_max) {
-  const size_t ms = (size_t)max_splits_for(kv_len_max);
-  return align256((size_t)n * H * ms * Dh * sizeof(float)) + align256((size_t)n * H * ms * 2 * sizeof(float));
+  if (r < total_q) varlen_row(cu_q, cu_k, nseg, causal, r, row_base[r], kv_len[r]);
 }
 
 // Largest group of query rows one workgroup takes: 8 MFMA rows (NR = QG * G),

@@ -213,6 +213,30 @@ def attn_varlen_rows(cu_q: torch.Tensor, cu_k: torch.Tensor, total_q: int, *, ca
     return kv_row_base, kv_len
 
 
+def attn_varlen(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu_q: torch.Tensor, cu_k: torch.Tensor, *,
+                max_k: int, causal: bool, scale: float | None = None) -> torch.Tensor:
+    """Packed varlen attention (wfd_attn_varlen; bf16): q (total_q, H, Dh),
+    k / v (total_k, Hkv, Dh), cu_q / cu_k int32 (nseg + 1,) on the device. The
+    tables and split partials live in a workspace of the call's own."""
+    _need_cuda(q, k, v, cu_q, cu_k)
+    _need(q.dim() == 3 and q.is_contiguous(), "q must be contiguous (n, H, Dh)")
+    n, H, Dh = q.shape
+    Hkv, cDh, _ = kv_layout(k, v)
+    _need(k.dim() == 3 and cDh == Dh and k.dtype == q.dtype, "q/k/v dtype or head_dim mismatch")
+    _need(cu_q.dtype == torch.int32 and cu_k.dtype == torch.int32 and cu_q.is_contiguous() and cu_k.is_contiguous()
+          and cu_q.numel() == cu_k.numel() and cu_q.numel() >= 1, "cu_q / cu_k: int32 (nseg + 1,)")
+    lib, nseg = _lib.load(), cu_q.numel() - 1
+    out = torch.empty_like(q)
+    ws_bytes = lib.wfd_attn_varlen_workspace_bytes(nseg, n, H, Hkv, Dh, int(max_k))
+    ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=q.device)
+    sc = 1.0 / math.sqrt(Dh) if scale is None else float(scale)
+    rc = lib.wfd_attn_varlen(q.data_ptr(), k.data_ptr(), v.data_ptr(), cu_q.data_ptr(), cu_k.data_ptr(),
+                             out.data_ptr(), nseg, n, H, Hkv, Dh, _dt(q), sc, int(max_k), 1 if causal else 0,
+                             ws.data_ptr(), ws_bytes, _stream())
+    _lib.check(rc, "wfd_attn_varlen")
+    return out
+
+
 def attn_prefill(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, seg_row_base: torch.Tensor,
                  seg_q_start: torch.Tensor, seg_pos0: torch.Tensor, *, max_seg_len: int, scale: float | None = None,
                  out: torch.Tensor | None = None) -> torch.Tensor:
