@@ -270,6 +270,73 @@ def test_linear_row_invariant(gpu, dtype, N):
     assert torch.equal(a[0], b[0])
 
 
+@pytest.mark.parametrize("K", [128, 384, 2048, 2176, 5632])
+@pytest.mark.parametrize("N", [528, 4112])
+def test_linear_block_kernel_same_bits(gpu, N, K):
+    """The block kernel's three workgroup shapes at the edges of their rows (32
+    and 64 and 128 row groups with a row too many or too few), a ragged last
+    tile group (33 and 257 tiles), one and several chunks per sub-slice, fewer
+    half chunks than ring stages, odd chunk counts: every row has the few-row
+    kernel's bits, for bf16 and fp32 outputs, SwiGLU, row scales, gathered
+    rows, pitched x, and outputs whose row pitch does not keep 4-element
+    alignment (33 tiles are the stream kernel's up to 256 rows)."""
+    g = torch.Generator().manual_seed(N + K)
+    n = 641
+    X = torch.randn(n, K + 32, generator=g).to(torch.bfloat16).to(gpu)[:, :K]
+    W = (0.05 * torch.randn(N, K, generator=g)).to(torch.bfloat16).to(gpu)
+    Wp, Ws = ops.pack_linear(W), ops.pack_linear(W, swiglu=True)
+    scale = (torch.rand(n, generator=g) + 0.5).to(gpu)
+    rs = lambda i, m: ops.RowScale(D=2048, eps=1e-6, two=True, scale=scale[i: i + m].contiguous())  # noqa: E731
+    print(f"[linear block] N={N} K={K}", flush=True)
+
+    def few(fn):
+        return torch.cat([fn(X[i: i + 16], i, min(16, n - i)) for i in range(0, n, 16)])
+
+    ref = few(lambda x, i, m: ops.linear(x, Wp))
+    ref32 = few(lambda x, i, m: ops.linear(x, Wp, out_dtype=torch.float32))
+    refs = few(lambda x, i, m: ops.linear(x, Ws, swiglu=True, rowscale=rs(i, m)))
+    rows = torch.randperm(n, generator=g)[:300].to(torch.int32).to(gpu)
+    for m in (33, 64, 65, 127, 129, 257, 300, 600, 641):
+        assert torch.equal(ops.linear(X, Wp, n=m), ref[:m]), m
+        assert torch.equal(ops.linear(X, Wp, n=m, out_dtype=torch.float32), ref32[:m]), m
+        assert torch.equal(ops.linear(X, Ws, n=m, swiglu=True, rowscale=rs(0, m)), refs[:m]), m
+    assert torch.equal(ops.linear(X, Wp, x_rows=rows), ref[rows.long()])
+    for dt, r in ((torch.bfloat16, ref), (torch.float32, ref32)):
+        out = torch.zeros(n, N + 1, dtype=dt, device=gpu)
+        ops.linear(X, Wp, out=out, out_dtype=dt)
+        assert torch.equal(out[:, :N], r) and not out[:, N:].any()
+    assert rel_err(_np(ref32[:40]), ok.linear(_np(X[:40]), _np(W))) <= 1e-3
+
+
+@pytest.mark.parametrize("H,Hkv,Dh,blocks", [(32, 32, 64, True), (24, 8, 128, False)])
+def test_linear_block_kernel_rope_append(gpu, H, Hkv, Dh, blocks):
+    """QKV + RoPE + append through the block kernel's three workgroup shapes:
+    q and every cache row have the few-row kernel's bits."""
+    g = torch.Generator().manual_seed(H)
+    n, K, S = 600, 2048, 700
+    N = (H + 2 * Hkv) * Dh
+    X = torch.randn(n, K, generator=g).to(torch.bfloat16).to(gpu)
+    Wp = ops.pack_linear((0.05 * torch.randn(N, K, generator=g)).to(torch.bfloat16).to(gpu))
+    pos = torch.randint(0, S, (n,), generator=g).to(torch.int32).to(gpu)
+    cos, sin = torch.rand(S, Dh // 2, generator=g).to(gpu), torch.rand(S, Dh // 2, generator=g).to(gpu)
+    fr = torch.randperm(S, generator=g)[:n].to(gpu)
+    scale = (torch.rand(n, generator=g) + 0.5).to(gpu)
+    shape = (1, Hkv, S, Dh) if blocks else (S, Hkv, Dh)
+    mk = lambda: torch.zeros(shape, dtype=torch.bfloat16, device=gpu)  # noqa: E731
+    print(f"[linear block rope] H={H} Hkv={Hkv} Dh={Dh}", flush=True)
+
+    def go(i, m, k, v):
+        rs = ops.RowScale(D=K, eps=1e-6, two=True, scale=scale[i: i + m].contiguous())
+        return ops.linear_qkv_rope_append(X[i: i + m], Wp, pos[i: i + m].contiguous(), cos, sin,
+                                          fr[i: i + m].contiguous(), k, v, H, Hkv, Dh, rowscale=rs)
+
+    for m in (40, 300, 600):
+        k0, v0, k1, v1 = mk(), mk(), mk(), mk()
+        q0 = torch.cat([go(i, min(16, m - i), k0, v0) for i in range(0, m, 16)])
+        q1 = go(0, m, k1, v1)
+        assert torch.equal(q0, q1) and torch.equal(k0, k1) and torch.equal(v0, v1), m
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("N,K", [(2048, 2048), (2048, 5632), (2048, 4096), (256, 1024), (512, 384), (128, 128)])
 def test_linear_split_k_same_bits(gpu, dtype, N, K):

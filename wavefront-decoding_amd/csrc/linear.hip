@@ -25,7 +25,7 @@
 // adds them in slice order); the sub-slices (at most 16) let a few-row launch
 // give each wave one run of chunks to sum in registers. Every sum starts at
 // +0 and so is never -0: adding a +0 for an empty (sub-)slice leaves its bits.
-// Five kernels honour the contract bit for bit:
+// Six kernels honour the contract bit for bit:
 //
 //  * wide (n <= 16): one 16-wave workgroup per tile (or column half of a
 //    tile), 8 waves when there are more than 512 tiles; wave w sums sub-slice
@@ -36,12 +36,15 @@
 //  * tile (n > 16, few row-block x tile pairs): a workgroup owns 64 rows of x
 //    and 2 tiles; each of its 4 waves walks the chunks in order for one
 //    16-row block of x and both tiles, with a two-stage register pipeline.
-//  * gemm (n > 16, many pairs): 64 rows x 2 or 4 tiles per workgroup, the
+//  * gemm (fp32, n > 16, many pairs): 64 rows x 2 or 4 tiles per workgroup, the
 //    tiles' weights staged once in LDS for the 4 waves, weights and x loaded
 //    two chunks ahead, an XCD-aware grid.
 //  * stream (n > 16, at most 256 tiles): 64 rows x 1 or 2 tiles per
 //    workgroup, weights and x moved global -> LDS by direct-to-LDS loads
 //    through a 4-stage ring (3 chunks in flight without registers).
+//  * block (bf16; n > 16 with more than 512 tiles, n > 32 with more than 256,
+//    else n > 256): 64 or 128 rows x 64 or 128 columns per workgroup, half-chunk
+//    stages through an LDS ring.
 //  * gemm, slice form (wfd_linear_partials): the gemm kernel over one slice
 //    of K per workgroup (grid y = slice), storing fp32 slice partials.
 //
@@ -1135,6 +1138,283 @@ __global__ __launch_bounds__(256) void linear_stream_kernel(const T* __restrict_
   }
 }
 
+// ---------------------------------------------------------------------------
+// block: NW waves (16 or 8), 32 RW rows x 16 CT (NW / RW) columns per
+// workgroup, 32 x 16 CT per wave (RW row groups x NW / RW column groups). For
+// launches that are matrix-core work: a byte loaded from L2 feeds 64-128 rows or
+// columns, where the 64-row gemm workgroup reads its x again for every 32-64
+// columns.
+//
+// K moves in half chunks (64 bf16 elements) global -> LDS with direct
+// loads (load16_lds) through a ring of NS stages: a half chunk of weights is
+// packed fragments as they lie in memory, a half chunk of x is 8 rows x 128
+// bytes per load, pieces XORed by half the row number so that a fragment read
+// (16 rows, one piece each) spreads over all banks (no conflicts counted).
+// Waits and barrier per stage as in the stream kernel, one stage earlier, so a
+// step's fragments are read while the step before it runs.
+//
+// What bounds it: the per-stage barrier and the loads. At 1500 rows x 5632
+// inputs x 2048 columns the matrix cores are busy 34 % of the time with 8 waves;
+// without MFMAs the launch takes 44 us, without loads 50, all of it 53; with 16
+// waves of half the columns each (four per SIMD to run through the others'
+// waits, a register set of 128) 49 us. Row by row, us before (stream / gemm
+// kernel) and now: gate|up + SwiGLU (11264 x 2048) at 64 / 112 / 192 / 512 / 1500 rows
+// 18 / 23 / 30 / 52 / 146 -> 14 / 18 / 24 / 44 / 109; q|k|v (6144 x 2048) 13.5 / 15 /
+// 21 / 29 / 77 -> 12 / 13 / 15 / 22 / 59; 2048 x 5632 at 512 / 1500 rows 46 / 128 ->
+// 31 / 49; lm_head (32000 x 2048) at 64 / 112 / 512 rows 32 / 43 / 127 -> 28 / 34 / 91.
+//
+// The product is formed transposed (weights as the A operand, x as B: the same
+// dot products, so the same bits): a lane ends with 4 consecutive columns of
+// one row, which it stores at once, a RoPE pair in its own registers.
+//
+// ONE: one chunk per sub-slice (K of at most 16 chunks): the chunk partial is
+// the sub-slice sum ((0 + c) added to a sum that is never -0 leaves the bits of
+// c added to it), so no sub-slice registers.
+
+template <typename T>
+__device__ __forceinline__ const T* half_x_ptr(const T* __restrict__ x, const int32_t* __restrict__ x_rows,
+                                               int64_t ldx, int row, int piece, int n) {
+  const int m = row < n ? row : n - 1;  // rows past the last read the last row; never stored
+  return x + (int64_t)(x_rows ? x_rows[m] : m) * ldx + piece * Chunk<T>::V;
+}
+
+// Output columns c0 .. c0 + 3 (of tile g) of one row, v in column order; `up`
+// (SwiGLU): the up values of gate columns c0 .. c0 + 3.
+template <typename TO, int EPI>
+__device__ __forceinline__ void store_out4(TO* __restrict__ y, int64_t ldy, const RopeArgs& ra, int row, int pos,
+                                           int64_t ro, int g, int c0, const float (&v)[4], const float (&up)[4]) {
+  float o[4];
+  TO* dst;
+  if constexpr (EPI == kEpiSwiGLU) {
+    if (c0 >= 8) return;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = (v[e] / (1.0f + expf(-v[e]))) * up[e];
+    dst = y + (int64_t)row * ldy + 8 * g + c0;
+  } else if constexpr (EPI == kEpiRope) {
+    int dbase;
+    const int head = tile_head(ra, g, dbase);
+    const int d = dbase + c0;
+    if (head >= ra.H + ra.Hkv) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = v[e];
+      dst = (TO*)ra.v_cache + ro + (head - ra.H - ra.Hkv) * kv_head_stride(ra) + d;
+    } else {
+      const int64_t t = (int64_t)pos * (ra.Dh >> 1) + (d >> 1);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {  // store_rope's rotation of the pair (2 j, 2 j + 1)
+        const float c = ra.cos_t[t + j], s = ra.sin_t[t + j];
+        const float x0 = Elem<TO>::round(v[2 * j]), x1 = Elem<TO>::round(v[2 * j + 1]);
+        o[2 * j] = fmaf(x0, c, -(x1 * s));
+        o[2 * j + 1] = fmaf(x0, s, x1 * c);
+      }
+      dst = head < ra.H ? (TO*)ra.q_out + ((int64_t)row * ra.H + head) * ra.Dh + d
+                        : (TO*)ra.k_cache + ro + (head - ra.H) * kv_head_stride(ra) + d;
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = v[e];
+    dst = y + (int64_t)row * ldy + 16 * g + c0;
+  }
+  if (((uintptr_t)dst & (4 * sizeof(TO) - 1)) == 0) {
+    if constexpr (sizeof(TO) == 2)
+      *reinterpret_cast<uint2*>(dst) = uint2{f32x2_to_bf16x2_bits(o[0], o[1]), f32x2_to_bf16x2_bits(o[2], o[3])};
+    else
+      *reinterpret_cast<f32x4*>(dst) = f32x4{o[0], o[1], o[2], o[3]};
+  } else {  // a row pitch or base that is not a multiple of 4 elements
+#pragma unroll
+    for (int e = 0; e < 4; ++e) Elem<TO>::store(dst + e, o[e]);
+  }
+}
+
+template <typename T, typename TO, int EPI, int NW, int RW, int CT, int NS, bool ONE>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW / 4))) void linear_block_kernel(
+    const T* __restrict__ x, const int32_t* __restrict__ x_rows, int64_t ldx, const T* __restrict__ W,
+    TO* __restrict__ y, int64_t ldy, int n, int K, int tiles, const RopeArgs ra, const float* __restrict__ rscale) {
+  constexpr int V = LinTraits<T>::V;
+  constexpr int KH = LinTraits<T>::KC / 2;  // elements per half chunk
+  constexpr int CW = NW / RW;      // column groups
+  constexpr int BT = CW * CT;               // weight tiles per workgroup
+  constexpr int BR = 32 * RW;               // rows per workgroup
+  constexpr int NWL = 2 * BT;               // 1 KB weight fragments (tile, step) per half chunk
+  constexpr int NXL = BR / 8;               // 1 KB x loads per half chunk
+  constexpr int WPW = NWL / NW, XPW = NXL / NW;  // loads per wave
+  static_assert(NWL % NW == 0 && NXL % NW == 0, "every wave issues the same loads");
+  constexpr int LPS = WPW + XPW;
+  static_assert(NS >= 4, "a stage in use, one landed, one landing, one being issued");
+  __shared__ __align__(16) u32x4 ws[NS][NWL][64];
+  __shared__ __align__(16) u32x4 xs[NS][NXL][64];
+
+  // XCD-aware mapping as xcd_block: the row blocks of a tile group on one XCD
+  const int RB = (n + BR - 1) / BR;
+  const int j0 = blockIdx.x / kXcds;
+  const int rbk = j0 % RB;
+  const int tg = (j0 / RB) * kXcds + blockIdx.x % kXcds;
+  if (tg * BT >= tiles) return;  // padding workgroup (uniform, before any barrier)
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int grp = lane >> 4;
+  const int rw = wave / CW, cw = wave % CW;
+  const int row0 = rbk * BR + 32 * rw;
+  const bool rows = row0 < n;  // uniform over the wave
+  const int P = K / LinTraits<T>::KC;
+
+  const T* wsrc[WPW];
+#pragma unroll
+  for (int i = 0; i < WPW; ++i) {
+    const int f = wave * WPW + i;  // (tile f / 2, step f % 2 of the half)
+    const int g = tg * BT + f / 2;
+    wsrc[i] = W + packed_off<T>(g < tiles ? g : tiles - 1, 0, P, lane) + (int64_t)(f % 2) * 64 * V;
+  }
+  const T* xsrc[XPW];
+#pragma unroll
+  for (int i = 0; i < XPW; ++i) {
+    const int r = 8 * (wave * XPW + i) + (lane >> 3);
+    xsrc[i] = half_x_ptr<T>(x, x_rows, ldx, rbk * BR + r, (lane & 7) ^ ((r >> 1) & 7), n);
+  }
+  const int H2 = 2 * P;  // half chunks; half h: steps 2 (h % 2), 2 (h % 2) + 1 of chunk h / 2
+  auto issue = [&](int h) {
+    const int st = h % NS;
+#pragma unroll
+    for (int i = 0; i < WPW; ++i) load16_lds(wsrc[i] + (int64_t)h * 2 * 64 * V, &ws[st][wave * WPW + i][0]);
+#pragma unroll
+    for (int i = 0; i < XPW; ++i) load16_lds(xsrc[i] + (int64_t)h * KH, &xs[st][wave * XPW + i][0]);
+  };
+#pragma unroll
+  for (int u = 0; u < NS - 1; ++u)
+    if (u < H2) issue(u);
+
+  SliceWalk walk(P, 0);
+  f32x4 sub[2][CT], sl[2][CT], tot[2][CT];
+  f32x4 acc0[2][CT], acc1[2][CT];  // chunk partials: even chunks, odd chunks
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int t = 0; t < CT; ++t) tot[a][t] = sl[a][t] = sub[a][t] = acc1[a][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // fragments of step s of half chunk h
+  auto read = [&](u32x4 (&xf)[2], u32x4 (&wf)[CT], int h, int s) {
+    const int st = h % NS;
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+      const int r = lane & 15;  // row of the 16-row block; unit of (row, piece): 8 row + (piece ^ row / 2)
+      xf[a] = (&xs[st][4 * rw + 2 * a][0])[8 * r + ((4 * s + grp) ^ (r >> 1))];
+    }
+#pragma unroll
+    for (int t = 0; t < CT; ++t) wf[t] = ws[st][2 * (cw * CT + t) + s][lane];
+  };
+  auto mma = [&](f32x4 (&acc)[2][CT], const u32x4 (&xf)[2], const u32x4 (&wf)[CT], bool first) {
+#pragma unroll
+    for (int t = 0; t < CT; ++t)
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+        acc[a][t] = mfma_step<T>(wf[t], xf[a], first ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[a][t]);
+  };
+  // a chunk partial into the innermost running sum (its slice's with ONE, else
+  // its sub-slice's), and what the end of chunk p closes
+  auto add = [&](const f32x4 (&acc)[2][CT]) {
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int t = 0; t < CT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) (ONE ? sl : sub)[a][t][r] += acc[a][t][r];
+  };
+  auto into = [&](f32x4 (&to)[2][CT], f32x4 (&from)[2][CT]) {
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int t = 0; t < CT; ++t) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) to[a][t][r] += from[a][t][r];
+        from[a][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+  };
+  auto close = [&](int p) {
+    const int lvl = walk.end(p);
+    if (!ONE && lvl >= 1) into(sl, sub);
+    if (lvl == 2) into(tot, sl);
+  };
+  // stage h + 1 has landed for every wave, and every wave's reads of stage
+  // h - 1 have completed: its slot takes half chunk h + NS - 1
+  auto turn = [&](int h) {
+    if (h + NS - 1 <= H2)
+      wait_vmem_barrier<(NS - 3) * LPS>();
+    else
+      wait_vmem_barrier<0>();
+    if (h + NS - 1 < H2) issue(h + NS - 1);
+  };
+  // Each step's fragments are read while the step before it runs (past the
+  // last half chunk: unused values of some stage), and chunk p - 1's partial is
+  // added while chunk p's first half runs: one addition per MFMA, in the
+  // 16 cycles that the matrix core takes.
+  u32x4 xa[2], wa[CT], xb[2], wb[CT];
+  auto chunk = [&](f32x4 (&acc)[2][CT], const f32x4 (&prev)[2][CT], int p) {
+    turn(2 * p);
+    read(xb, wb, 2 * p, 1);
+    mma(acc, xa, wa, true);
+    add(prev);
+    read(xa, wa, 2 * p + 1, 0);
+    mma(acc, xb, wb, false);
+    if constexpr (sizeof(T) == 2) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        __builtin_amdgcn_sched_group_barrier(0x100, 2 + CT, 0);  // LDS reads
+#pragma unroll
+        for (int i = 0; i < 2 * CT; ++i) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);     // MFMA
+          __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);     // VALU
+        }
+      }
+    }
+    turn(2 * p + 1);
+    if (p > 0) close(p - 1);
+    read(xb, wb, 2 * p + 1, 1);
+    mma(acc, xa, wa, false);
+    read(xa, wa, 2 * p + 2, 0);
+    mma(acc, xb, wb, false);
+  };
+  if (H2 >= NS - 1)
+    wait_vmem_barrier<(NS - 2) * LPS>();
+  else
+    wait_vmem_barrier<0>();
+  read(xa, wa, 0, 0);
+  int p = 0;
+  for (; p + 1 < P; p += 2) {
+    chunk(acc0, acc1, p);  // before chunk 0: adds zeros
+    chunk(acc1, acc0, p + 1);
+  }
+  if (p < P) {
+    chunk(acc0, acc1, p);
+    add(acc0);
+  } else {
+    add(acc1);
+  }
+  close(P - 1);
+  if (!rows) return;  // after the last barrier; every load of this wave has completed
+#pragma unroll
+  for (int a = 0; a < 2; ++a) {
+    const int row = row0 + 16 * a + (lane & 15);
+    const int rc = row < n ? row : n - 1;
+    const float sc = rscale ? rscale[rc] : 1.f;  // a folded norm pair's row scale
+    int pos = 0;
+    int64_t ro = 0;
+    if constexpr (EPI == kEpiRope) {
+      pos = rope_row_pos(ra, rc);
+      ro = rope_row_off(ra, rc);
+    }
+#pragma unroll
+    for (int t = 0; t < CT; ++t) {
+      const int g = tg * BT + cw * CT + t;
+      if (g >= tiles) continue;  // uniform over the wave
+      float v[4], up[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = rscale ? mul_rn(tot[a][t][r], sc) : tot[a][t][r];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) up[r] = EPI == kEpiSwiGLU ? __shfl_xor(v[r], 32, 64) : 0.f;  // columns c + 8
+      if (row < n) store_out4<TO, EPI>(y, ldy, ra, row, pos, ro, g, 4 * grp, v, up);
+    }
+  }
+}
+
 // The few-row regime's launch shape for n rows, `tiles` 16-column tiles and R
 // chunks per sub-slice.
 struct WidePlan {
@@ -1154,6 +1434,48 @@ static WidePlan wide_plan(int n, int tiles, int R, bool swiglu) {
   w.ww8 = !w.half && tiles > kResidentWide && R == 1;
   w.groups = w.wide ? (w.half ? 2 * tiles : tiles) : 0;
   return w;
+}
+
+// Workgroup shape of the block kernel for a launch, or none. Times of one round
+// of workgroups at K = 2048 (us): 128 x 128 (16 waves) 18.5, 128 x 64 13.5 -- one per
+// CU by their LDS -- and 64 x 64, two per CU, 11.5 for up to 256 workgroups and
+// 17 for up to 512; the shape with the fewest rounds by that measure was the
+// fastest, or within 3 %, at 64-1500 rows x 128-2000 tiles. With at most
+// kStreamMaxTiles tiles the stream kernel's one- and two-tile workgroups fill
+// more CUs up to 256 rows (2048 x 5632 at 64 / 192 / 512 rows: stream 18 / 24 / 46,
+// block 30 / 30 / 31 us); at 32 rows or fewer and up to 512 tiles the tile kernel
+// streams the weights without barriers (q|k|v 11.7 against 12.4 us; gate|up and
+// lm_head are faster here: 16.5 -> 14.7, 30.5 -> 25.3 us).
+enum BlockShape : int { kBlockNone = 0, kBlock128x128, kBlock128x64, kBlock64x64 };
+
+static int block_shape(int n, int tiles) {
+  if ((tiles <= kStreamMaxTiles && n <= 256) || (tiles <= kGemmMinBlockTiles && n <= 32)) return kBlockNone;
+  const long rb128 = (n + 127) / 128, rb64 = (n + 63) / 64, g8 = (tiles + 7) / 8, g4 = (tiles + 3) / 4;
+  const long a = 37 * ((rb128 * g8 + 255) / 256);
+  const long b = 27 * ((rb128 * g4 + 255) / 256);
+  const long c = rb64 * g4 <= 256 ? 23 : 34 * ((rb64 * g4 + 511) / 512);
+  return a <= b && a <= c ? kBlock128x128 : b <= c ? kBlock128x64 : kBlock64x64;
+}
+
+template <typename TO, int EPI>
+static void launch_block(int shape, const void* x, const int32_t* xr, int64_t ldx, const void* W, void* y, int64_t ldy,
+                         int n, int K, int tiles, bool one, const RopeArgs& ra, const float* rsc, hipStream_t st) {
+#define WFD_BLOCK(NW, RW, CT, ONE)                                                                              \
+  hipLaunchKernelGGL((linear_block_kernel<bf16_t, TO, EPI, NW, RW, CT, 4, ONE>),                               \
+                     dim3(xcd_grid((n + 32 * RW - 1) / (32 * RW), (tiles + NW / RW * CT - 1) / (NW / RW * CT))), \
+                     dim3(64 * NW), 0, st, (const bf16_t*)x, xr, ldx, (const bf16_t*)W, (TO*)y, ldy, n, K, tiles, \
+                     ra, rsc)
+  if (shape == kBlock128x128) {
+    if (one) WFD_BLOCK(16, 4, 2, true);
+    else WFD_BLOCK(16, 4, 2, false);
+  } else if (shape == kBlock128x64) {
+    if (one) WFD_BLOCK(8, 4, 2, true);
+    else WFD_BLOCK(8, 4, 2, false);
+  } else {
+    if (one) WFD_BLOCK(8, 2, 1, true);
+    else WFD_BLOCK(8, 2, 1, false);
+  }
+#undef WFD_BLOCK
 }
 
 template <typename T, typename TO, int EPI>
@@ -1189,6 +1511,13 @@ static void launch_linear(const void* x, const int32_t* xr, int64_t ldx, const v
 #undef WFD_WIDE
     const float* rsc = rs.scale;  // many rows: the scales precomputed (group sums are few-row only)
     const int rb = (n + 63) / 64;
+    if constexpr (std::is_same<T, bf16_t>::value) {
+      const int bs = block_shape(n, tiles);
+      if (bs != kBlockNone) {
+        launch_block<TO, EPI>(bs, x, xr, ldx, W, y, ldy, n, K, tiles, R == 1, ra, rsc, st);
+        return;
+      }
+    }
     if (tiles <= kStreamMaxTiles) {
       // few weight tiles: each workgroup walks all of K, so its chunk chain is
       // the launch's critical path; keep kStreamStages - 1 chunks in flight.
@@ -1203,31 +1532,27 @@ static void launch_linear(const void* x, const int32_t* xr, int64_t ldx, const v
                            (const T*)x, xr, ldx, (const T*)W, (TO*)y, ldy, n, K, pair_off, tiles, ra, rsc);
       return;
     }
-    // few (row block, tile) pairs, or at most 32 rows where four-tile gemm
-    // workgroups would not cover the CUs: every wave streams its own weights,
-    // no barriers (gate|up at 17-32 rows: 16.1-17.1 -> 14.0-14.9 us; lm_head,
-    // with 500 gemm workgroups, stays on the gemm)
-    if (rb * tiles <= kGemmMinBlockTiles || (n <= 32 && (tiles + 3) / 4 < 256)) {
+    // few (row block, tile) pairs (bf16: at most 32 rows): every wave streams its
+    // own weights, no barriers
+    if (std::is_same<T, bf16_t>::value || rb * tiles <= kGemmMinBlockTiles || (n <= 32 && (tiles + 3) / 4 < 256)) {
       constexpr int NB = 2;
       hipLaunchKernelGGL((linear_tile_kernel<T, TO, EPI, NB>), dim3(rb, (tiles + NB - 1) / NB), dim3(256), 0, st,
                          (const T*)x, xr, ldx, (const T*)W, (TO*)y, ldy, n, K, pair_off, tiles, ra, rsc);
       return;
     }
-    // weights through LDS, shared by the 4 waves: 4 tiles per workgroup
-    // while that still leaves >= 256 workgroups (128 for the epilogues
-    // without the RoPE operand tables), else 2. lm_head at 64 rows: 500
-    // four-tile workgroups 34 us, 1000 two-tile ones 42 us; gate|up at 64
-    // rows: 176 four-tile ones 16.4 us, 352 two-tile ones 17.8 us (in the
-    // bs=32 decode); Wqkv + RoPE at 128 rows keeps 2 (192 four-tile
-    // workgroups: 21.1 -> 24.5 us, the epilogue's tables cost registers per
-    // tile). Eight tiles per workgroup were slower in the decode for every
-    // one-launch shape (Wqkv + RoPE at 192 rows 28 -> 48 us).
-    if (rb * ((tiles + 3) / 4) >= (EPI == kEpiRope ? 256 : 128))
-      hipLaunchKernelGGL((linear_gemm_kernel<T, TO, EPI, 4, false>), dim3(xcd_grid(rb, (tiles + 3) / 4)), dim3(256), 0,
-                         st, (const T*)x, xr, ldx, (const T*)W, (TO*)y, ldy, n, K, pair_off, tiles, ra, nullptr, rsc);
-    else
-      hipLaunchKernelGGL((linear_gemm_kernel<T, TO, EPI, 2, false>), dim3(xcd_grid(rb, (tiles + 1) / 2)), dim3(256), 0,
-                         st, (const T*)x, xr, ldx, (const T*)W, (TO*)y, ldy, n, K, pair_off, tiles, ra, nullptr, rsc);
+    // fp32: weights through LDS, shared by the 4 waves: 4 tiles per workgroup
+    // while that still leaves >= 256 workgroups (128 for the epilogues without the
+    // RoPE operand tables, which cost registers per tile), else 2
+    if constexpr (!std::is_same<T, bf16_t>::value) {
+      if (rb * ((tiles + 3) / 4) >= (EPI == kEpiRope ? 256 : 128))
+        hipLaunchKernelGGL((linear_gemm_kernel<T, TO, EPI, 4, false>), dim3(xcd_grid(rb, (tiles + 3) / 4)), dim3(256),
+                           0, st, (const T*)x, xr, ldx, (const T*)W, (TO*)y, ldy, n, K, pair_off, tiles, ra, nullptr,
+                           rsc);
+      else
+        hipLaunchKernelGGL((linear_gemm_kernel<T, TO, EPI, 2, false>), dim3(xcd_grid(rb, (tiles + 1) / 2)), dim3(256),
+                           0, st, (const T*)x, xr, ldx, (const T*)W, (TO*)y, ldy, n, K, pair_off, tiles, ra, nullptr,
+                           rsc);
+    }
   }
 }
 
