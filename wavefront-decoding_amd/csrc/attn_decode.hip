@@ -156,6 +156,14 @@ __global__ __launch_bounds__(64 * NW) void attn_split_kernel(const T* __restrict
     for (int s = 0; s < NDS; ++s) qf[s] = real ? ld16(qp + s * KSTEP) : zero16();
   }
 
+  // The group's rows hold MFMA rows [0, nr): a group of fewer than QG rows skips
+  // the per-row work of the others (uniform branches; their values are never
+  // stored). A coda's 28 four-row groups x 16 heads over 128-1200 keys, Dh 128:
+  // 77 -> 66 us. Loading the next tile under this one's P.V (K through LDS, 40
+  // VGPRs spilled) took 93 us.
+  const int nr = __builtin_amdgcn_readfirstlane(qn * G);
+  auto live = [&](int m) { return QG == 1 || m < nr; };
+
   // running softmax state of this wave per row: max (log2 domain), sum, output
   float mrun[NR], lrun[NR], o[NR][V];
 #pragma unroll
@@ -236,9 +244,10 @@ __global__ __launch_bounds__(64 * NW) void attn_split_kernel(const T* __restrict
       mt4[r] = mt;
     }
     float corr[NR];
-    float mnew4[4];
+    float mnew4[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
 #pragma unroll
     for (int m = 0; m < NR; ++m) {
+      if (!live(m)) continue;
       const float mt = __uint_as_float(__shfl(__float_as_uint(mt4[m % 4]), 16 * (m / 4), 64));
       const float mnew = fmaxf(mrun[m], mt);
       corr[m] = (mrun[m] == -INFINITY) ? 0.f : exp2f(mrun[m] - mnew);
@@ -262,6 +271,7 @@ __global__ __launch_bounds__(64 * NW) void attn_split_kernel(const T* __restrict
     }
 #pragma unroll
     for (int m = 0; m < NR; ++m) {
+      if (!live(m)) continue;
       const float lt = __uint_as_float(__shfl(__float_as_uint(lt4[m % 4]), 16 * (m / 4), 64));
       lrun[m] = fmaf(lrun[m], corr[m], lt);
     }
@@ -282,19 +292,38 @@ __global__ __launch_bounds__(64 * NW) void attn_split_kernel(const T* __restrict
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 
     // P.V on the VALU: lane owns V columns [dseg*V, dseg*V+V) of keys RG*k + vg
+    if constexpr (QG == 1) {
 #pragma unroll
-    for (int m = 0; m < NR; ++m)
+      for (int m = 0; m < NR; ++m)
 #pragma unroll
-      for (int e = 0; e < V; ++e) o[m][e] *= corr[m];
+        for (int e = 0; e < V; ++e) o[m][e] *= corr[m];
 #pragma unroll
-    for (int k = 0; k < KPL; ++k) {
-      float v[V];
-      Elem<T>::unpack(vf[k], v);
+      for (int k = 0; k < KPL; ++k) {
+        float v[V];
+        Elem<T>::unpack(vf[k], v);
+#pragma unroll
+        for (int m = 0; m < NR; ++m) {
+          const float p = p_lds[wave][m][vg * KPL + k];
+#pragma unroll
+          for (int e = 0; e < V; ++e) o[m][e] = fmaf(p, v[e], o[m][e]);
+        }
+      }
+    } else {  // row by row (the same sums), so that a row that is not there costs one branch
+      float v[KPL][V];
+#pragma unroll
+      for (int k = 0; k < KPL; ++k) Elem<T>::unpack(vf[k], v[k]);
 #pragma unroll
       for (int m = 0; m < NR; ++m) {
-        const float p = p_lds[wave][m][vg * KPL + k];
+        if (!live(m)) continue;
+        float p[KPL];
 #pragma unroll
-        for (int e = 0; e < V; ++e) o[m][e] = fmaf(p, v[e], o[m][e]);
+        for (int k = 0; k < KPL; ++k) p[k] = p_lds[wave][m][vg * KPL + k];
+#pragma unroll
+        for (int e = 0; e < V; ++e) o[m][e] *= corr[m];
+#pragma unroll
+        for (int k = 0; k < KPL; ++k)
+#pragma unroll
+          for (int e = 0; e < V; ++e) o[m][e] = fmaf(p[k], v[k][e], o[m][e]);
       }
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -302,16 +331,16 @@ __global__ __launch_bounds__(64 * NW) void attn_split_kernel(const T* __restrict
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
 #pragma unroll
-  for (int sh = LPR; sh < 64; sh <<= 1)
+  for (int m = 0; m < NR; ++m) {
+    if (!live(m)) continue;
 #pragma unroll
-    for (int m = 0; m < NR; ++m)
+    for (int sh = LPR; sh < 64; sh <<= 1)
 #pragma unroll
       for (int e = 0; e < V; ++e) o[m][e] += __shfl_xor(o[m][e], sh, 64);
-  if (vg == 0) {
-#pragma unroll
-    for (int m = 0; m < NR; ++m)
+    if (vg == 0) {
 #pragma unroll
       for (int e = 0; e < V; ++e) o_lds[wave][m][dseg * V + e] = o[m][e];
+    }
   }
   if (lane == 0) {
 #pragma unroll
