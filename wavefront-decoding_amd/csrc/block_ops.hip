@@ -303,20 +303,24 @@ static void launch_add_rmsnorm(int dtype, const void* a, const int32_t* a_rows, 
                               stream);
 }
 
-// Folded norm pairs, the row form (wfd_norm_prep; wfd_prep_t in wfd.h). One
-// wave per row, the lane layout of add_rmsnorm_kernel: lane L = c + 16 j
-// holds, at step s, the elements of chunk c at s KSTEP + j V -- for bf16 one
+// Folded norm pairs, the row form (wfd_norm_prep; wfd_prep_t in wfd.h). Four
+// waves per row, wave s = step s of the lane layout of add_rmsnorm_kernel: lane
+// L = c + 16 j holds, at step s, the elements of chunk c at s KSTEP + j V -- for bf16 one
 // whole 8-column group, for fp32 half of one (the other half in lane L ^ 16).
 // Each element is wfd_linear_prep's epilogue value (prep_value), each group
 // sum the same tree, and the lane adds its groups in step order before the
 // butterfly -- the order a consumer adds the group sums wfd_linear_prep
-// stores (fold_slot), so the scales are equal bit for bit. SPLIT: y is the
+// stores (fold_slot), so the scales are equal bit for bit: the waves leave their
+// step's group sums in LDS and every wave adds all four, in step order. At 16-512
+// rows of 2048 the launch is a chain of one row's work (loads, ~800 vector
+// instructions with four steps in one wave), which four waves shorten:
+// 112 rows with four slices 6.7 -> 4.8 us. SPLIT: y is the
 // in-order slice sum of wfd_linear_partials (the linear's output before its
 // rounding); else y = a[i] (already rounded). r (when kept) and A are stored
 // as soon as they are formed, the scales after the sums; XOUT keeps r for
 // h = round((r * s_a) * wa), the first norm's output, written to rows h_rows.
 template <typename T, bool SPLIT, bool RES, bool XOUT>
-__global__ __launch_bounds__(256) void norm_prep_kernel(const T* __restrict__ a, int64_t lda,
+__global__ __launch_bounds__(64 * kChunkSteps) void norm_prep_kernel(const T* __restrict__ a, int64_t lda,
                                                         const float* __restrict__ part, int64_t slice_stride,
                                                         int nslices, const wfd_prep_t pp, int two, float eps,
                                                         float* __restrict__ scale_out, float* __restrict__ s_out,
@@ -325,123 +329,113 @@ __global__ __launch_bounds__(256) void norm_prep_kernel(const T* __restrict__ a,
   constexpr int V = Chunk<T>::V;
   constexpr int KSTEP = Chunk<T>::KSTEP;
   constexpr int KC = Chunk<T>::KC;
-  const int i = blockIdx.x * (blockDim.x >> 6) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  __shared__ float2 groups[kChunkSteps][64];  // the lanes' group sums, by step
+  const int i = blockIdx.x;
+  const int s = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // this wave's step
   const int lane = threadIdx.x & 63;
   const int c = lane & 15;
   const int j = lane >> 4;
-  if (i >= n) return;  // no barriers below
   const int P = D / KC;
   const int p = c < P ? c : P - 1;  // lanes past the last chunk re-read it (their values are never used)
   const bool live = fold_lane_live<T>(lane, P);
   const T* wa_t = (const T*)pp.wa;
   const T* wb_t = (const T*)pp.wb;
   const bool prep = pp.a_out != nullptr;  // uniform
-  [[maybe_unused]] float r[kChunkSteps][V];
-  float gr[kChunkSteps], gu[kChunkSteps];
+  float rv[V];
   float s_in = 1.f;
   if constexpr (RES) {
     if (pp.s_in) s_in = pp.s_in[i];
   }
-  // every load of the row first, then the arithmetic and the stores: the
-  // stores cannot be shown not to alias the loads, so loads issued after one
-  // would wait for it, one HBM round trip per step
+  // every load first, then the arithmetic and the stores (which cannot be shown
+  // not to alias the loads). A wave reads only the elements it writes, so rows
+  // may be updated in place
   constexpr int YL = SPLIT ? kSplitMaxSlices * (V / 4) : 1;
   const u32x4 one = Elem<T>::pack_ones();
-  u32x4 yraw[kChunkSteps][YL], rraw[kChunkSteps], wiraw[kChunkSteps], waraw[kChunkSteps], wbraw[kChunkSteps];
+  const int64_t off = (int64_t)p * KC + s * KSTEP + j * V;
+  u32x4 yraw[YL], rraw = one, wiraw = one;
+  if constexpr (SPLIT) {
 #pragma unroll
-  for (int s = 0; s < kChunkSteps; ++s) {
-    const int64_t off = (int64_t)p * KC + s * KSTEP + j * V;
-    if constexpr (SPLIT) {
+    for (int q = 0; q < kSplitMaxSlices; ++q) {
+      const float* src = part + q * slice_stride + (int64_t)i * D + off;
 #pragma unroll
-      for (int q = 0; q < kSplitMaxSlices; ++q) {
-        const float* src = part + q * slice_stride + (int64_t)i * D + off;
-#pragma unroll
-        for (int h = 0; h < V / 4; ++h) yraw[s][q * (V / 4) + h] = q < nslices ? ld16(src + 4 * h) : u32x4{0, 0, 0, 0};
-      }
-    } else {
-      yraw[s][0] = ld16(a + (int64_t)i * lda + off);
+      for (int h = 0; h < V / 4; ++h) yraw[q * (V / 4) + h] = q < nslices ? ld16(src + 4 * h) : u32x4{0, 0, 0, 0};
     }
-    rraw[s] = wiraw[s] = one;
-    if constexpr (RES) {
-      rraw[s] = ld16((const T*)pp.r_in + (int64_t)i * pp.ld_in + off);
-      if (pp.w_in) wiraw[s] = ld16((const T*)pp.w_in + off);
-    }
-    waraw[s] = wa_t ? ld16(wa_t + off) : one;
-    wbraw[s] = prep ? ld16(wb_t + off) : one;
+  } else {
+    yraw[0] = ld16(a + (int64_t)i * lda + off);
   }
+  if constexpr (RES) {
+    rraw = ld16((const T*)pp.r_in + (int64_t)i * pp.ld_in + off);
+    if (pp.w_in) wiraw = ld16((const T*)pp.w_in + off);
+  }
+  const u32x4 waraw = wa_t ? ld16(wa_t + off) : one;
+  const u32x4 wbraw = prep ? ld16(wb_t + off) : one;
+  float y[V];
+  if constexpr (SPLIT) {
+    // slices in order from +0 (slices past nslices load as +0)
 #pragma unroll
-  for (int s = 0; s < kChunkSteps; ++s) {
-    const int64_t off = (int64_t)p * KC + s * KSTEP + j * V;
-    float y[V];
-    if constexpr (SPLIT) {
-      // slices in order from +0 (slices past nslices load as +0)
+    for (int e = 0; e < V; ++e) y[e] = 0.f;
 #pragma unroll
-      for (int e = 0; e < V; ++e) y[e] = 0.f;
+    for (int q = 0; q < kSplitMaxSlices; ++q) {
 #pragma unroll
-      for (int q = 0; q < kSplitMaxSlices; ++q) {
+      for (int h = 0; h < V / 4; ++h) {
 #pragma unroll
-        for (int h = 0; h < V / 4; ++h) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) y[4 * h + e] += __uint_as_float(yraw[s][q * (V / 4) + h][e]);
-        }
+        for (int e = 0; e < 4; ++e) y[4 * h + e] += __uint_as_float(yraw[q * (V / 4) + h][e]);
       }
-    } else {
-      Elem<T>::unpack(yraw[s][0], y);
     }
-    float rin[V], win[V], wa[V], wb[V];
-    Elem<T>::unpack(rraw[s], rin);
-    Elem<T>::unpack(wiraw[s], win);
-    Elem<T>::unpack(waraw[s], wa);
-    Elem<T>::unpack(wbraw[s], wb);
-    float rv[V], Av[V], sr[V], su[V];
+  } else {
+    Elem<T>::unpack(yraw[0], y);
+  }
+  float rin[V], win[V], wa[V], wb[V];
+  Elem<T>::unpack(rraw, rin);
+  Elem<T>::unpack(wiraw, win);
+  Elem<T>::unpack(waraw, wa);
+  Elem<T>::unpack(wbraw, wb);
+  float Av[V], sr[V], su[V];
 #pragma unroll
-    for (int e = 0; e < V; ++e) {
-      const PrepVal pv = prep_value<T>(y[e], RES, rin[e], s_in, win[e], wa[e], wb[e]);
-      rv[e] = pv.r;
-      Av[e] = pv.A;
-      sr[e] = pv.sr;
-      su[e] = pv.su;
-    }
-    if constexpr (XOUT) {
+  for (int e = 0; e < V; ++e) {
+    const PrepVal pv = prep_value<T>(y[e], RES, rin[e], s_in, win[e], wa[e], wb[e]);
+    rv[e] = pv.r;
+    Av[e] = pv.A;
+    sr[e] = pv.sr;
+    su[e] = pv.su;
+  }
+  if (c < P) {
+    if (pp.r_out) *reinterpret_cast<u32x4*>((T*)pp.r_out + (int64_t)i * pp.ld_out + off) = Elem<T>::pack(rv);
+    if (prep) *reinterpret_cast<u32x4*>((T*)pp.a_out + (int64_t)i * pp.ld_a + off) = Elem<T>::pack(Av);
+  }
+  // the group's tree: ((c0+c1)+(c2+c3))+((c4+c5)+(c6+c7))
+  float tr = tree4(sr[0], sr[1], sr[2], sr[3]);
+  float tu = tree4(su[0], su[1], su[2], su[3]);
+  if constexpr (V == 8) {
+    tr = add_rn(tr, tree4(sr[4], sr[5], sr[6], sr[7]));
+    tu = add_rn(tu, tree4(su[4], su[5], su[6], su[7]));
+  } else {  // the group's other half sits in lane L ^ 16
+    tr = add_rn(tr, __shfl_xor(tr, 16, 64));
+    tu = add_rn(tu, __shfl_xor(tu, 16, 64));
+  }
+  groups[s][lane] = live ? float2{tr, tu} : float2{0.f, 0.f};
+  __syncthreads();  // also: every wave has read s_in[i] before s_out[i] is written
+  float gr[kChunkSteps], gu[kChunkSteps];
 #pragma unroll
-      for (int e = 0; e < V; ++e) r[s][e] = rv[e];
-    }
-    if (c < P) {
-      if (pp.r_out) *reinterpret_cast<u32x4*>((T*)pp.r_out + (int64_t)i * pp.ld_out + off) = Elem<T>::pack(rv);
-      if (prep) *reinterpret_cast<u32x4*>((T*)pp.a_out + (int64_t)i * pp.ld_a + off) = Elem<T>::pack(Av);
-    }
-    // the group's tree: ((c0+c1)+(c2+c3))+((c4+c5)+(c6+c7))
-    float tr = tree4(sr[0], sr[1], sr[2], sr[3]);
-    float tu = tree4(su[0], su[1], su[2], su[3]);
-    if constexpr (V == 8) {
-      tr = add_rn(tr, tree4(sr[4], sr[5], sr[6], sr[7]));
-      tu = add_rn(tu, tree4(su[4], su[5], su[6], su[7]));
-    } else {  // the group's other half sits in lane L ^ 16
-      tr = add_rn(tr, __shfl_xor(tr, 16, 64));
-      tu = add_rn(tu, __shfl_xor(tu, 16, 64));
-    }
-    gr[s] = live ? tr : 0.f;
-    gu[s] = live ? tu : 0.f;
+  for (int t = 0; t < kChunkSteps; ++t) {
+    const float2 g = groups[t][lane];
+    gr[t] = g.x;
+    gu[t] = g.y;
   }
   float srow, surow;
   fold_sums(gr, gu, srow, surow);
   float s_a, scale;
   pair_scale(srow, surow, D, eps, two != 0, s_a, scale);
-  if (prep && lane == 0) {
+  if (prep && threadIdx.x == 0) {
     scale_out[i] = scale;
     if (s_out) s_out[i] = s_a;
   }
   if constexpr (XOUT) {
     const int64_t orow = h_rows ? h_rows[i] : i;
+    float h[V];
 #pragma unroll
-    for (int s = 0; s < kChunkSteps; ++s) {
-      const int64_t off = (int64_t)p * KC + s * KSTEP + j * V;
-      float wa[V], h[V];
-      Elem<T>::unpack(waraw[s], wa);
-#pragma unroll
-      for (int e = 0; e < V; ++e) h[e] = norm_value<T>(r[s][e], s_a, wa[e]);
-      if (c < P) *reinterpret_cast<u32x4*>(h_out + orow * ldh + off) = Elem<T>::pack(h);
-    }
+    for (int e = 0; e < V; ++e) h[e] = norm_value<T>(rv[e], s_a, wa[e]);
+    if (c < P) *reinterpret_cast<u32x4*>(h_out + orow * ldh + off) = Elem<T>::pack(h);
   }
 }
 
@@ -449,8 +443,7 @@ template <typename T, bool SPLIT, bool RES, bool XOUT>
 static void launch_norm_prep_t(const void* a, int64_t lda, const float* part, int64_t slice_stride, int nslices,
                                const wfd_prep_t& pp, int two, float eps, float* scale_out, float* s_out, void* h_out,
                                const int32_t* h_rows, int64_t ldh, int n, int D, hipStream_t stream) {
-  const int rpw = n >= kNormRowsPerCuLaunch ? 4 : 1;  // as add_rmsnorm: rows spread one per CU below 1024
-  const dim3 grid((n + rpw - 1) / rpw), block(64 * rpw);
+  const dim3 grid(n), block(64 * kChunkSteps);
   hipLaunchKernelGGL((norm_prep_kernel<T, SPLIT, RES, XOUT>), grid, block, 0, stream, (const T*)a, lda, part,
                      slice_stride, nslices, pp, two, eps, scale_out, s_out, (T*)h_out, h_rows, ldh, n, D);
 }
