@@ -199,6 +199,17 @@ def _bucket(n: int) -> int:
     return b
 
 
+# Prompt rows up to which each bf16 linear of the prompt pass stays on the packed
+# kernels (q|k|v with its RoPE + append epilogue, gate|up with its SwiGLU) although
+# the library GEMM is at hand: us per call on the 2048-d model at 128 / 256 / 512 /
+# 640 / 768 / 1024 rows, packed against library (+ epilogue launch): q|k|v 15 / 18 /
+# 24 / 25 / 39 / 45 against 33 / 34 / 34 / 35 / 37 / 41; proj 11 / 12 / 13 / 15 / 15 / 16
+# against 19 throughout; gate|up 19 / 24 / 44 / 45 / 60 / 65 against 30 / 31 / 36 / 38 /
+# 48 / 58; down 18 / 25 / 31 / 37 against 19 / 21 / 26 / 33; adapter 14 / 19 / 23 / 28
+# against 19 / 19 / 21 / 24. Below ~20 us the library call is bound by its host side.
+_PACKED_PROMPT_ROWS = {"Wqkv": 640, "proj": 1024, "fc": 256, "mlp_proj": 128, "adapter": 256}
+
+
 class LoopedModel:
     """Device-resident looped LM running unions of rows through libwfd."""
 
@@ -224,10 +235,10 @@ class LoopedModel:
         # same bits as the one-launch linear, more workgroups per launch
         self.split_rows = _SPLIT_ROWS
         self.W = {}
-        # the prompt pass (prefill_seq) runs its linears as plain library GEMMs
-        # over row-major copies of the block weights: its rows are computed once
-        # and never compared bit for bit with decode rows, and at hundreds to
-        # tens of thousands of rows the library GEMM is 2-9x faster
+        # the prompt pass (prefill_seq) runs its larger linears as plain library
+        # GEMMs over row-major copies of the block weights: its rows are computed
+        # once and never compared bit for bit with decode rows, and from some
+        # hundreds of rows on (_PACKED_PROMPT_ROWS) the library GEMM is faster
         self.dense_prompt = dense_prompt
         self.Wd: dict[str, torch.Tensor] = {}
         for k, v in weights.items():
@@ -363,11 +374,13 @@ class LoopedModel:
         kernel (rows grouped by slot at consecutive positions) instead of the
         per-row decode kernel; `group_first` groups decode rows that share a
         slot (one prefix read per group, same bits). `dense` (the prompt pass)
-        runs the four linears as library GEMMs over the row-major weights, with
-        the RoPE/append and SwiGLU epilogues as their own kernels."""
+        runs the linears beyond the packed kernels' row range (_library_rows) as
+        library GEMMs over the row-major weights, with the RoPE/append and
+        SwiGLU epilogues as their own kernels."""
         c, W = self.cfg, self.W
         x, h = sc["x"], sc["h"]
-        if dense:
+        lib = lambda leaf: dense and self._library_rows(leaf, n)  # noqa: E731
+        if lib("Wqkv"):
             qkv = torch.mm(h[:n], self.Wd[prefix + "Wqkv"].t(), out=sc["qkv"][:n])
             q = ops.qkv_rope_append(qkv, pos_d, self.rope_cos, self.rope_sin, fr_d, cache.flat_k, cache.flat_v,
                                     c.n_heads, c.n_kv_heads, c.head_dim, q_out=sc["q"][:n])
@@ -381,30 +394,30 @@ class LoopedModel:
         else:
             o = ops.attn_decode(q, cache.flat_k, cache.flat_v, rb_d, kvlen_d, kv_len_max=kv_len_max,
                                 out=sc["o"][:n], workspace=ws, group_first=group_first)
-        if dense:
+        if lib("proj"):
             a = torch.mm(o.view(n, -1), self.Wd[prefix + "proj"].t(), out=sc["a"][:n])
             ops.add_rmsnorm(a, W[prefix + "norm_2"], c.norm_eps, res=x, w2=W[prefix + "norm_3"], n=n, x_out=x,
                             h_out=h)
         else:
             self._linear_norm(o.view(n, -1), W[prefix + "proj"], n, sc, "a", W[prefix + "norm_2"], res=x,
                               w2=W[prefix + "norm_3"], x_out=x, h_out=h)
-        if dense:
+        if lib("fc"):
             gu = torch.mm(h[:n], self.Wd[prefix + "fc"].t(), out=sc["gu"][:n])
             u = ops.swiglu(gu, n=n, out=sc["u"][:n])
-            m = torch.mm(u, self.Wd[prefix + "mlp_proj"].t(), out=sc["m"][:n])
-            if next_norm is not None:
-                ops.add_rmsnorm(m, W[prefix + "norm_4"], c.norm_eps, res=x, w2=next_norm, n=n, x_out=x, h_out=h)
-            else:
-                ops.add_rmsnorm(m, W[prefix + "norm_4"], c.norm_eps, res=x, n=n, x_out=final_out,
-                                out_rows=final_rows)
         else:
             u = ops.linear(h, W[prefix + "fc"], n=n, out=sc["u"], swiglu=True)
-            if next_norm is not None:
-                self._linear_norm(u, W[prefix + "mlp_proj"], n, sc, "m", W[prefix + "norm_4"], res=x,
-                                  w2=next_norm, x_out=x, h_out=h)
-            else:
-                self._linear_norm(u, W[prefix + "mlp_proj"], n, sc, "m", W[prefix + "norm_4"], res=x,
-                                  x_out=final_out, out_rows=final_rows)
+        out = (dict(w2=next_norm, x_out=x, h_out=h) if next_norm is not None
+               else dict(x_out=final_out, out_rows=final_rows))
+        if lib("mlp_proj"):
+            m = torch.mm(u[:n], self.Wd[prefix + "mlp_proj"].t(), out=sc["m"][:n])
+            ops.add_rmsnorm(m, W[prefix + "norm_4"], c.norm_eps, res=x, n=n, **out)
+        else:
+            self._linear_norm(u, W[prefix + "mlp_proj"], n, sc, "m", W[prefix + "norm_4"], res=x, **out)
+
+    def _library_rows(self, leaf: str, n: int) -> bool:
+        """Whether the prompt pass runs this linear over n rows as a library
+        GEMM (with dense_prompt): beyond the packed kernels' range (bf16), or fp32."""
+        return self.dtype != torch.bfloat16 or n > _PACKED_PROMPT_ROWS[leaf]
 
     def _linear_norm(self, xin: torch.Tensor, Wp, n: int, sc, tmp: str, w1: torch.Tensor, *, x_rows=None,
                      keep=None, **norm) -> None:
@@ -415,7 +428,9 @@ class LoopedModel:
         core block's residual)."""
         lo, hi = self.split_rows
         eps = self.cfg.norm_eps
-        if lo <= n <= hi:
+        # above 128 rows the one-launch linear (proj 11-13 us) and a norm over its
+        # bf16 rows cost less than slices (12-14 us) and a norm over four fp32 ones
+        if lo <= n <= min(hi, 128):
             S = ops.linear_partials(xin, Wp, sc["part"], n=n, x_rows=x_rows)
             ops.add_rmsnorm_split(sc["part"], S, n, w1, eps, dtype=self.dtype, a_out=keep, **norm)
         else:
@@ -820,8 +835,8 @@ class LoopedModel:
     def prefill_seq(self, cache, b: int, token_ids) -> torch.Tensor:
         """Whole prompt of sequence b at positions [0, L): fills every slot's
         [0, L) and returns the last position's logits (V,) float32. Runs eagerly
-        with its own L-row scratch; with dense_prompt its linears are library
-        GEMMs (see __init__), the last position's lm_head row the packed kernel."""
+        with its own L-row scratch; with dense_prompt its larger linears are library
+        GEMMs (see __init__, _library_rows), the last position's lm_head row the packed kernel."""
         c, W = self.cfg, self.W
         ids = np.asarray(token_ids, dtype=np.int64).reshape(-1)
         L = len(ids)
@@ -859,7 +874,7 @@ class LoopedModel:
                         final_out=state[:, D:], segments=seg_l(i), dense=dense)
         state[:, :D].copy_(self._prompt_s0(L))
         for r in range(c.T_total):
-            if dense:
+            if dense and self._library_rows("adapter", L):
                 torch.mm(state, self.Wd["adapter"].t(), out=sc["x"][:L])
             else:
                 ops.linear(state, W["adapter"], n=L, out=sc["x"])
