@@ -15,6 +15,7 @@ import torch
 from oracle import kernels as ok
 from tests.conftest import rel_err
 from wavefront_decoding_amd import attention as A
+from wavefront_decoding_amd import ops
 
 pytestmark = pytest.mark.gpu
 
@@ -86,7 +87,8 @@ def test_attn_varlen_shared_rows(gpu, causal, H, Hkv, Dh):
     print(f"[attn_varlen shared rows] causal={causal} H={H} Hkv={Hkv} Dh={Dh}", flush=True)
     dev = [t.to(gpu) for t in (q, k, v)]
     cq, ck = torch.from_numpy(cu_q).to(gpu), torch.from_numpy(cu_k).to(gpu)
-    out = A.attn_varlen(*dev, cq, ck, max(a for a, _ in seg), max(b for _, b in seg), causal=causal)
+    shared = lambda q_, k_, v_, a, b, mk_: ops.attn_varlen(q_, k_, v_, a, b, max_k=mk_, causal=causal)  # noqa: E731
+    out = shared(*dev, cq, ck, max(b for _, b in seg))
     ref = np.zeros((n, H, Dh))
     ref[lead: int(cu_q[-1])] = _varlen_ref(q[lead:], k, v, cu_q - lead, cu_k, causal)[: int(cu_q[-1]) - lead]
     got = _np(out)
@@ -101,8 +103,29 @@ def test_attn_varlen_shared_rows(gpu, causal, H, Hkv, Dh):
     vs = torch.cat([dev[2][cu_k[i]: cu_k[i + 1]] for i in last] + [dev[2][:7]])
     kl = [seg[i][1] for i in last] + [7]
     off = lambda x: torch.tensor(np.concatenate([[0], np.cumsum(x)]), dtype=torch.int32, device=gpu)  # noqa: E731
-    alone = A.attn_varlen(qs, ks, vs, off([1] * len(last) + [2]), off(kl), 2, max(kl), causal=causal)
+    alone = shared(qs, ks, vs, off([1] * len(last) + [2]), off(kl), max(kl))
     assert torch.equal(alone[: len(last)], out[rows])
+
+
+@pytest.mark.parametrize("rows,causal", [(3, True), (70, True), (70, False)])
+def test_attn_varlen_routes_agree(gpu, rows, causal):
+    """attn_varlen and non-causal attn_dense on both sides of the choice of
+    kernel (three rows a segment: the decode kernel; 70: the shared-rows one)
+    against the decode kernel's rows: each is within bf16 rounding of float64."""
+    H, Hkv, Dh, segs, Tk = 4, 4, 128, 5, 130
+    g = torch.Generator().manual_seed(rows)
+    q, k, v = (torch.randn(segs * r, h, Dh, generator=g).to(torch.bfloat16).to(gpu)
+               for r, h in ((rows, H), (Tk, Hkv), (Tk, Hkv)))
+    cq, ck = (torch.arange(segs + 1, dtype=torch.int32, device=gpu) * t for t in (rows, Tk))
+    assert A._shared_rows(q, k, segs * rows, segs, Tk) == (rows == 70)
+    rb, kl = ops.attn_varlen_rows(cq, ck, segs * rows, causal=causal)
+    ref = ops.attn_decode(q, k, v, rb, kl, kv_len_max=Tk).float()
+    outs = [A.attn_varlen(q, k, v, cq, ck, rows, Tk, causal=causal)]
+    if not causal:
+        outs.append(A.attn_dense(q.view(segs, rows, H, Dh), k.view(segs, Tk, Hkv, Dh), v.view(segs, Tk, Hkv, Dh),
+                                 causal=False).view_as(q))
+    for out in outs:  # two bf16 roundings of the same value
+        assert (out.float() - ref).norm() <= 2.0 ** -8 * ref.norm()
 
 
 def test_attn_varlen_shared_rows_special_values(gpu):
@@ -114,10 +137,10 @@ def test_attn_varlen_shared_rows_special_values(gpu):
     n, H, Dh = 60, 2, 128
     q, k, v = (torch.randn(n, H, Dh, generator=g).to(torch.bfloat16).to(gpu) for _ in range(3))
     cu = torch.tensor([0, n], dtype=torch.int32, device=gpu)
-    plain = A.attn_varlen(q, k, v, cu, cu, n, n, causal=True)
+    plain = ops.attn_varlen(q, k, v, cu, cu, max_k=n, causal=True)
     v[40, 0, 5] = float("inf")
     v[50, 1, 7] = float("nan")
-    got = A.attn_varlen(q, k, v, cu, cu, n, n, causal=True)
+    got = ops.attn_varlen(q, k, v, cu, cu, max_k=n, causal=True)
     assert torch.equal(got[:32], plain[:32])
     assert torch.isinf(got[40:, 0, 5]).all() and torch.isnan(got[50:, 1, 7]).all()
     clean = torch.ones_like(got, dtype=torch.bool)

@@ -9,15 +9,15 @@ runs a HIP kernel of libwfd.so on torch's current stream:
 
   attn_dense      bf16 causal with Tq <= Tk (a prompt, bottom-right aligned):
                   the MFMA prefill kernel (wfd_attn_prefill), one segment per
-                  batch row; any other bf16 call with Tq > 1: the varlen kernel
+                  batch row; other bf16 calls of many rows: the varlen kernel
                   (wfd_attn_varlen), one segment per batch row; otherwise the
                   decode kernel (wfd_attn_decode) with one (row base, key
                   count) entry per query row
   attn_cutoff_multi  the decode kernel with key count = qpos + 1
-  attn_varlen     bf16 with more rows than segments: the varlen kernel, whose
-                  workgroups read a key once for up to 32 / (H / Hkv) rows of
-                  its segment; otherwise (a row per segment, fp32) the decode
-                  kernel over the packed K / V (token-major), its row tables
+  attn_varlen     bf16 with at least four rows per segment and rows enough
+                  (_shared_rows): the varlen kernel, whose workgroups read a
+                  key once for up to 32 / (H / Hkv) rows of its segment;
+                  otherwise the decode kernel over the packed K / V (token-major), its row tables
                   expanded from cu_q / cu_k on the device
                   (wfd_attn_varlen_rows). Nothing is read back to the host
   attn_varlen_q1_padded  attn_varlen with one query row per segment (the
@@ -104,12 +104,23 @@ def _prefill_segments(B: int, Tq: int, Tk: int, device):
     return _cached(("prefill", B, Tq, Tk, str(device)), build)
 
 
-def _shared_rows(q: torch.Tensor, k: torch.Tensor) -> bool:
+def _shared_rows(q: torch.Tensor, k: torch.Tensor, total_q: int, nseg: int, max_k: int) -> bool:
     """Whether the kernel that reads a key once for all rows of a segment
-    (wfd_attn_varlen) takes these heads: bf16, Dh 64 / 128, 1, 2 or 4 query
-    heads per kv head."""
+    (wfd_attn_varlen) takes this call: bf16, Dh 64 / 128, 1, 2 or 4 query heads
+    per kv head, and rows enough to gain by it. The decode kernel's workgroups
+    (one per row, kv head and 1024 keys) repeat the segment's reads but spread
+    over more CUs: it wins below four rows a segment (48 segments of 2 rows x
+    1000 keys x 16 heads: 88 against 111 us; of 4 rows 134 against 112) and while its
+    launch is at most two rounds of resident workgroups, two per CU, or with Dh
+    64 or four query heads (one per CU by LDS) one round (one segment of 16 / 64
+    rows x 1000 keys x 16 heads: 13 / 33 against 23 / 24 us; 4 segments of 16 / 32
+    rows, 16 heads over 4 kv heads: 20 / 36 against 24 / 24 us)."""
+    if total_q < 4 * nseg or q.dtype != torch.bfloat16 or k.dtype != torch.bfloat16:
+        return False
     H, Dh, Hkv = q.shape[-2], q.shape[-1], k.shape[-2]
-    return q.dtype == k.dtype == torch.bfloat16 and Dh in (64, 128) and Hkv > 0 and H in (Hkv, 2 * Hkv, 4 * Hkv)
+    if Dh not in (64, 128) or Hkv <= 0 or H not in (Hkv, 2 * Hkv, 4 * Hkv):
+        return False
+    return total_q * Hkv * ((max_k + 1023) // 1024) > (256 if H == 4 * Hkv else 511 if Dh == 64 else 1023)
 
 
 def _dense_offsets(B: int, Tq: int, Tk: int, device):
@@ -134,7 +145,7 @@ def attn_dense(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, causal: boo
     if causal and Tq > 1 and Tq <= Tk and q.dtype == torch.bfloat16 and Dh in (64, 128):
         rb, qs, p0 = _prefill_segments(B, Tq, Tk, q.device)
         out = ops.attn_prefill(qf, kf, vf, rb, qs, p0, max_seg_len=Tq, scale=_scale(Dh))
-    elif Tq > 1 and _shared_rows(q, k):
+    elif Tq > 1 and _shared_rows(q, k, B * Tq, B, max(Tk, 1)):
         cq, ck = _dense_offsets(B, Tq, Tk, q.device)
         out = ops.attn_varlen(qf, kf, vf, cq, ck, max_k=max(Tk, 1), causal=causal, scale=_scale(Dh))
     else:
@@ -175,7 +186,7 @@ def attn_varlen(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu_q: torch.T
         raise _lib.WfdError("attn_varlen: q (total_q, H, Dh), k / v (total_k, Hkv, Dh)")
     cq = cu_q.to(device=q.device, dtype=torch.int32).contiguous()
     ck = cu_k.to(device=q.device, dtype=torch.int32).contiguous()
-    if total_q >= cq.numel() and _shared_rows(q, k):  # some segment brings more than one row
+    if _shared_rows(q, k, total_q, cq.numel() - 1, max(int(max_k), 1)):
         return ops.attn_varlen(q.contiguous(), k.contiguous(), v.contiguous(), cq, ck, max_k=max(int(max_k), 1),
                                causal=causal, scale=_scale(Dh))
     rb, kl = ops.attn_varlen_rows(cq, ck, total_q, causal=causal)

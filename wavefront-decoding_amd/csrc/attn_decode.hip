@@ -419,14 +419,18 @@ constexpr int group_max_rows(int G) { return G >= kAttnGroupRows ? 1 : kAttnGrou
 // Measured on the 2048-d model's layer tick (8 rows, 512-778 keys): 15.2 ->
 // 13.7 us; 2 rows 12.3 -> 10.7 us; 4 and 8 parts are slower (21 / 35 us),
 // since the repeated K reads reach HBM again whatever the dispatch order.
+// Four query heads per kv head leave one workgroup per CU (86 KB of LDS, two
+// below that), where more than 256 parts run a second round: 192 workgroups of
+// 16 segments x 3 rows x 1000 keys took 37 us in two parts each, 22 us whole.
 // Every column keeps the unsplit arithmetic, so the split changes no bits.
 constexpr int kAttnFillWorkgroups = 256;
 constexpr int kAttnMaxVSplit = 2;
 
-static int attn_vsplit(int ms, int Hkv, int n, int DH) {
+static int attn_vsplit(int ms, int Hkv, int n, int DH, int G) {
   const int64_t base = (int64_t)ms * Hkv * n;
+  const int64_t fill = G == 4 ? kAttnFillWorkgroups / 2 + 1 : kAttnFillWorkgroups;
   int vs = 1;
-  while (vs < kAttnMaxVSplit && base * vs < kAttnFillWorkgroups && DH % (16 * vs) == 0) vs *= 2;
+  while (vs < kAttnMaxVSplit && base * vs < fill && DH % (16 * vs) == 0) vs *= 2;
   return vs;
 }
 
@@ -438,7 +442,7 @@ static void launch_attn(const void* q, const void* kc, const void* vc, const int
   constexpr int TK = DH == 64 ? 64 : 32;  // key tile that fits the registers
   constexpr int NW = 8;  // waves per workgroup: 8 beat 4 and 16 on every measured shape
   constexpr int QG = group_max_rows(G);
-  const int vs = attn_vsplit(ms, Hkv, n, DH);
+  const int vs = attn_vsplit(ms, Hkv, n, DH, G);
   if (gf)
     hipLaunchKernelGGL((attn_split_kernel<T, DH, G, QG, NW, TK>), dim3(ms, Hkv, n * vs), dim3(64 * NW), 0, st,
                        (const T*)q, (const T*)kc, (const T*)vc, rb, kl, gf, po, pml, (T*)out, H, Hkv, ms, scale_log2,

@@ -43,7 +43,7 @@
 //    workgroup, weights and x moved global -> LDS by direct-to-LDS loads
 //    through a 4-stage ring (3 chunks in flight without registers).
 //  * block (bf16; n > 16 with more than 512 tiles, n > 32 with more than 256,
-//    else n > 256): 64 or 128 rows x 64 or 128 columns per workgroup, half-chunk
+//    else n > 256 and work enough): 64 or 128 rows x 64 or 128 columns per workgroup, half-chunk
 //    stages through an LDS ring.
 //  * gemm, slice form (wfd_linear_partials): the gemm kernel over one slice
 //    of K per workgroup (grid y = slice), storing fp32 slice partials.
@@ -1442,15 +1442,16 @@ static WidePlan wide_plan(int n, int tiles, int R, bool swiglu) {
 // 17 for up to 512; the shape with the fewest rounds by that measure was the
 // fastest, or within 3 %, at 64-1500 rows x 128-2000 tiles. With at most
 // kStreamMaxTiles tiles the stream kernel's one- and two-tile workgroups fill
-// more CUs up to 256 rows (2048 x 5632 at 64 / 192 / 512 rows: stream 18 / 24 / 46,
+// more CUs up to 256 rows and below 160 of the 64 x 64 workgroups (2048 x 5632 at 64 / 192 / 512 rows: stream 18 / 24 / 46,
 // block 30 / 30 / 31 us); at 32 rows or fewer and up to 512 tiles the tile kernel
 // streams the weights without barriers (q|k|v 11.7 against 12.4 us; gate|up and
 // lm_head are faster here: 16.5 -> 14.7, 30.5 -> 25.3 us).
 enum BlockShape : int { kBlockNone = 0, kBlock128x128, kBlock128x64, kBlock64x64 };
 
 static int block_shape(int n, int tiles) {
-  if ((tiles <= kStreamMaxTiles && n <= 256) || (tiles <= kGemmMinBlockTiles && n <= 32)) return kBlockNone;
   const long rb128 = (n + 127) / 128, rb64 = (n + 63) / 64, g8 = (tiles + 7) / 8, g4 = (tiles + 3) / 4;
+  if ((tiles <= kStreamMaxTiles && (n <= 256 || rb64 * g4 < 160)) || (tiles <= kGemmMinBlockTiles && n <= 32))
+    return kBlockNone;
   const long a = 37 * ((rb128 * g8 + 255) / 256);
   const long b = 27 * ((rb128 * g4 + 255) / 256);
   const long c = rb64 * g4 <= 256 ? 23 : 34 * ((rb64 * g4 + 511) / 512);
