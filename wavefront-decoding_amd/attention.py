@@ -225,18 +225,28 @@ def _fused_qkv_weight(attn):
     return cached[1]
 
 
+def _token_tables(B: int, T: int, device):
+    """(positions 0..T-1 of every batch row, int32; row numbers, int64) of B * T
+    packed tokens. One pair per shape, built on the host and copied; a stream
+    under capture gets its own, which the graph then owns."""
+    if torch.cuda.is_current_stream_capturing():
+        return (torch.arange(T, dtype=torch.int32, device=device).repeat(B),
+                torch.arange(B * T, dtype=torch.int64, device=device))
+    return _cached(("tokens", B, T, str(device)), lambda: (torch.arange(T, dtype=torch.int32).repeat(B).to(device),
+                                                           torch.arange(B * T, dtype=torch.int64).to(device)))
+
+
 def _rope_tables(freqs, B: int, T: int, Dh: int, device):
-    """(cos, sin, per-row positions) for the QKV epilogue from the
+    """(cos, sin, per-row positions, or None for 0..T-1 of every batch row) for the QKV epilogue from the
     reference's complex freqs_cis (row t = position t's rotation, the same
     for every batch row) or from a (cos, sin, positions) tuple."""
     if torch.is_tensor(freqs) and freqs.is_complex():
         f = freqs.reshape(-1, Dh // 2)
         if f.shape[0] != T:
             raise _lib.WfdError(f"compute_qkv: freqs_cis holds {f.shape[0]} positions for T={T}")
-        f = f.to(device)
-        cos = f.real.to(torch.float32).contiguous()
-        sin = f.imag.to(torch.float32).contiguous()
-        pos = torch.arange(T, dtype=torch.int32, device=device)
+        # both parts in one launch
+        cos, sin = torch.view_as_real(f.to(device).resolve_conj()).permute(2, 0, 1).to(torch.float32).contiguous()
+        return cos, sin, None
     else:
         cos, sin, positions = freqs
         if isinstance(positions, int):
@@ -287,6 +297,7 @@ def compute_qkv(attn, x: torch.Tensor, freqs, ve=None, config=None):
     cos, sin, pos = _rope_tables(freqs, B, T, Dh, x.device)
     kbuf = torch.empty(n, Hkv, Dh, dtype=x.dtype, device=x.device)
     vbuf = torch.empty_like(kbuf)
-    rows = torch.arange(n, dtype=torch.int64, device=x.device)
+    tokens, rows = _token_tables(B, T, x.device)
+    pos = tokens if pos is None else pos
     q = ops.linear_qkv_rope_append(xf, W, pos, cos, sin, rows, kbuf, vbuf, H, Hkv, Dh)
     return q.view(B, T, H, Dh), kbuf.view(B, T, Hkv, Dh), vbuf.view(B, T, Hkv, Dh)

@@ -207,7 +207,7 @@ def _bucket(n: int) -> int:
 # against 19 throughout; gate|up 19 / 24 / 44 / 45 / 60 / 65 against 30 / 31 / 36 / 38 /
 # 48 / 58; down 18 / 25 / 31 / 37 against 19 / 21 / 26 / 33; adapter 14 / 19 / 23 / 28
 # against 19 / 19 / 21 / 24. Below ~20 us the library call is bound by its host side.
-_PACKED_PROMPT_ROWS = {"Wqkv": 640, "proj": 1024, "fc": 256, "mlp_proj": 128, "adapter": 256}
+_PACKED_PROMPT_ROWS = {"Wqkv": 640, "proj": 640, "fc": 256, "mlp_proj": 128, "adapter": 256}
 
 
 class LoopedModel:
