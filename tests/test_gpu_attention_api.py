@@ -117,7 +117,7 @@ def test_attn_varlen_routes_agree(gpu, rows, causal):
     q, k, v = (torch.randn(segs * r, h, Dh, generator=g).to(torch.bfloat16).to(gpu)
                for r, h in ((rows, H), (Tk, Hkv), (Tk, Hkv)))
     cq, ck = (torch.arange(segs + 1, dtype=torch.int32, device=gpu) * t for t in (rows, Tk))
-    assert A._shared_rows(q, k, segs * rows, segs, Tk) == (rows == 70)
+    assert A._shared_rows(segs * rows, segs, Tk, H, Hkv, Dh) == (rows == 70)
     rb, kl = ops.attn_varlen_rows(cq, ck, segs * rows, causal=causal)
     ref = ops.attn_decode(q, k, v, rb, kl, kv_len_max=Tk).float()
     outs = [A.attn_varlen(q, k, v, cq, ck, rows, Tk, causal=causal)]

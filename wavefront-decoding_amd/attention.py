@@ -14,7 +14,7 @@ runs a HIP kernel of libwfd.so on torch's current stream:
                   decode kernel (wfd_attn_decode) with one (row base, key
                   count) entry per query row
   attn_cutoff_multi  the decode kernel with key count = qpos + 1
-  attn_varlen     bf16 with at least four rows per segment and rows enough
+  attn_varlen     bf16 with at least two rows per segment and rows enough
                   (_shared_rows): the varlen kernel, whose workgroups read a
                   key once for up to 32 / (H / Hkv) rows of its segment;
                   otherwise the decode kernel over the packed K / V (token-major), its row tables
@@ -104,23 +104,21 @@ def _prefill_segments(B: int, Tq: int, Tk: int, device):
     return _cached(("prefill", B, Tq, Tk, str(device)), build)
 
 
-def _shared_rows(q: torch.Tensor, k: torch.Tensor, total_q: int, nseg: int, max_k: int) -> bool:
+def _shared_rows(total_q: int, nseg: int, max_k: int, H: int, Hkv: int, Dh: int) -> bool:
     """Whether the kernel that reads a key once for all rows of a segment
-    (wfd_attn_varlen) takes this call: bf16, Dh 64 / 128, 1, 2 or 4 query heads
+    (wfd_attn_varlen) takes this bf16 call: Dh 64 / 128, 1, 2 or 4 query heads
     per kv head, and rows enough to gain by it. The decode kernel's workgroups
     (one per row, kv head and 1024 keys) repeat the segment's reads but spread
-    over more CUs: it wins below four rows a segment (48 segments of 2 rows x
-    1000 keys x 16 heads: 88 against 111 us; of 4 rows 134 against 112) and while its
-    launch is at most two rounds of resident workgroups, two per CU, or with Dh
-    64 or four query heads (one per CU by LDS) one round (one segment of 16 / 64
-    rows x 1000 keys x 16 heads: 13 / 33 against 23 / 24 us; 4 segments of 16 / 32
-    rows, 16 heads over 4 kv heads: 20 / 36 against 24 / 24 us)."""
-    if total_q < 4 * nseg or q.dtype != torch.bfloat16 or k.dtype != torch.bfloat16:
+    over more CUs: it wins below two rows a segment and while its launch is at
+    most one round of resident workgroups, two per CU, or one with Dh 64 or (a
+    little earlier) with four query heads, by LDS. us, decode against this
+    kernel: 16 heads, 4 segments of 8 / 16 rows x 1000 keys (512 / 1024 workgroups)
+    19 / 32 against 19 / 19, 48 segments of 2 rows 87 against 73; 16 heads over 4
+    kv heads, 16 segments of 2 / 4 / 8 rows x 1000 keys 22 / 22 / 39 against 19; 4 over
+    2 heads of 64, 16 segments of 8 / 16 rows (256 / 512) 12.5 / 16.2 against 13.7."""
+    if total_q < 2 * nseg or Dh not in (64, 128) or Hkv <= 0 or H not in (Hkv, 2 * Hkv, 4 * Hkv):
         return False
-    H, Dh, Hkv = q.shape[-2], q.shape[-1], k.shape[-2]
-    if Dh not in (64, 128) or Hkv <= 0 or H not in (Hkv, 2 * Hkv, 4 * Hkv):
-        return False
-    return total_q * Hkv * ((max_k + 1023) // 1024) > (256 if H == 4 * Hkv else 511 if Dh == 64 else 1023)
+    return total_q * Hkv * ((max_k + 1023) // 1024) > (256 if Dh == 64 else 191 if H == 4 * Hkv else 512)
 
 
 def _dense_offsets(B: int, Tq: int, Tk: int, device):
@@ -145,7 +143,7 @@ def attn_dense(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, causal: boo
     if causal and Tq > 1 and Tq <= Tk and q.dtype == torch.bfloat16 and Dh in (64, 128):
         rb, qs, p0 = _prefill_segments(B, Tq, Tk, q.device)
         out = ops.attn_prefill(qf, kf, vf, rb, qs, p0, max_seg_len=Tq, scale=_scale(Dh))
-    elif Tq > 1 and _shared_rows(q, k, B * Tq, B, max(Tk, 1)):
+    elif Tq > 1 and q.dtype == k.dtype == torch.bfloat16 and _shared_rows(B * Tq, B, max(Tk, 1), H, Hkv, Dh):
         cq, ck = _dense_offsets(B, Tq, Tk, q.device)
         out = ops.attn_varlen(qf, kf, vf, cq, ck, max_k=max(Tk, 1), causal=causal, scale=_scale(Dh))
     else:
@@ -186,7 +184,8 @@ def attn_varlen(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu_q: torch.T
         raise _lib.WfdError("attn_varlen: q (total_q, H, Dh), k / v (total_k, Hkv, Dh)")
     cq = cu_q.to(device=q.device, dtype=torch.int32).contiguous()
     ck = cu_k.to(device=q.device, dtype=torch.int32).contiguous()
-    if _shared_rows(q, k, total_q, cq.numel() - 1, max(int(max_k), 1)):
+    if q.dtype == k.dtype == torch.bfloat16 and _shared_rows(total_q, cq.numel() - 1, max(int(max_k), 1), H, k.shape[1],
+                                                             Dh):
         return ops.attn_varlen(q.contiguous(), k.contiguous(), v.contiguous(), cq, ck, max_k=max(int(max_k), 1),
                                causal=causal, scale=_scale(Dh))
     rb, kl = ops.attn_varlen_rows(cq, ck, total_q, causal=causal)

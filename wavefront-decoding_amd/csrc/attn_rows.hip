@@ -17,9 +17,11 @@
 // 1024-key split round-robin, each with its own LDS block and no barrier in the
 // loop; a tile's 16 KB are loaded into registers (whole key rows, 1 KB per
 // instruction) while the tile before it is computed. Two workgroups per CU fit
-// by LDS (75 KB each at Dh 128), so one streams while the other merges. That
-// shape takes 158 us (the tables 5, this kernel 145, the merge of splits 10;
-// 2.7 TB/s) against 720 us for the row form.
+// by LDS (80 KB each at Dh 128, Q's fragments among them: in registers they made
+// the loop spill), so one streams while the other merges. That shape takes 124
+// us (the tables 5, this kernel 111, the merge of splits 10; 3.5 TB/s) against
+// 720 us for the row form; what is left is the ragged last round of 1540
+// workgroups over 512 places. Two S^T chains instead of one changed nothing.
 //
 // Arithmetic: S^T = K Q^T and O^T = V^T P^T on v_mfma_f32_32x32x16_bf16, V^T
 // read from the row-major tile with the transposing LDS read, keys permuted
@@ -114,16 +116,17 @@ __global__ __launch_bounds__(64 * kRowsWaves) __attribute__((amdgpu_waves_per_eu
   constexpr int QT = kRowsCols / G;        // rows per tile
   constexpr int NDS = DH / 16;             // MFMA k-steps over Dh
   constexpr int NDB = DH / 32;             // 32-row blocks of O^T
-  constexpr int KP = DH + 8;               // padded LDS row of K (elements)
-  constexpr int VRP = DH + 32;             // ... of V: spreads a transposing read over all banks
+  constexpr int VRP = DH + 32;             // padded LDS row of V (elements): spreads a transposing read over all banks
   constexpr int CPR = DH / V;              // 16-byte pieces of a key row
   constexpr int NCH = kRowsKeys * CPR / 64;  // K (and V) pieces per lane per tile
   constexpr int PW = NDB * 16 + 2;         // floats a lane parks for the merge
-  constexpr int kWaveLds = kRowsKeys * (KP + VRP) * (int)sizeof(bf16_t);
+  constexpr int kWaveLds = kRowsKeys * (DH + VRP) * (int)sizeof(bf16_t);
   static_assert(NW * kWaveLds >= NW * PW * 64 * (int)sizeof(float), "park area");
+  static_assert(NDS % NW == 0, "Q fragments staged by wave");
   static_assert(NDB <= NW && kRowsCols % G == 0, "merge split");
-  static_assert(kRowsKeys * KP * sizeof(bf16_t) >= kRowsKeys * 32 * sizeof(float), "P in the K tile's LDS");
+  static_assert(kRowsKeys * DH * sizeof(bf16_t) >= kRowsKeys * 32 * sizeof(float), "P in the K tile's LDS");
   __shared__ __align__(16) unsigned char lds[NW * kWaveLds];
+  __shared__ __align__(16) u32x4 q_lds[NDS][64];  // Q fragments: 32 registers a lane fewer, or the loop spills
 
   const int g = blockIdx.x % Hkv;
   const int tile = blockIdx.x / Hkv;
@@ -162,24 +165,31 @@ __global__ __launch_bounds__(64 * kRowsWaves) __attribute__((amdgpu_waves_per_eu
   const __amdgpu_buffer_rsrc_t vr = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(vc + hb), (short)0, span,
                                                                       0x00020000);
   bf16_t* const kl = reinterpret_cast<bf16_t*>(lds + wave * kWaveLds);
-  bf16_t* const vl = kl + kRowsKeys * KP;
+  bf16_t* const vl = kl + kRowsKeys * DH;
+  // K rows unpadded, 16-byte pieces XORed by the row: 16 rows' reads of one piece
+  // (and a row's 16 stores) touch every bank once
+  auto k_at = [](int key, int piece) {
+    return (key * CPR + (piece ^ (CPR == 16 ? key & 15 : (key >> 1) & (CPR - 1)))) * V;
+  };
 
   // Q as the MFMA B operand: column col, dims 16 k + 8 hf + (0..7)
-  u32x4 qf[NDS];
   {
     const bf16_t* qp = q + ((int64_t)row * H + head) * DH + hf * V;
 #pragma unroll
-    for (int k = 0; k < NDS; ++k) qf[k] = ld16(qp + k * 16);
+    for (int i = 0; i < NDS / NW; ++i) {
+      const int k = wave * (NDS / NW) + i;
+      q_lds[k][lane] = ld16(qp + k * 16);
+    }
   }
   // key (within a tile) of MFMA row col: the permutation above
   const int krow = 16 * ((col >> 3) >> 1) + 8 * ((col >> 2) & 1) + 4 * ((col >> 3) & 1) + (col & 3);
 
   u32x4 kreg[NCH], vreg[NCH];
+  const uint32_t lane_off = (uint32_t)(lane / CPR) * rsb + (uint32_t)(lane % CPR) * 16u;
   auto fetch = [&](int t) {
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
-      const int c = lane + 64 * i;
-      const uint32_t off = (uint32_t)(t * kRowsKeys + c / CPR) * rsb + (uint32_t)(c % CPR) * 16u;
+      const uint32_t off = lane_off + (uint32_t)(t * kRowsKeys + i * (64 / CPR)) * rsb;
       kreg[i] = buf_ld16(kr, off);
       vreg[i] = buf_ld16(vr, off);
     }
@@ -221,6 +231,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) __attribute__((amdgpu_waves_per_eu
   };
 
   fetch(wave);
+  __syncthreads();  // q_lds
   for (int t = wave; t < nt; t += NW) {  // uniform over the wave; no barrier in the loop
     // the LDS executes one wave's accesses in order: the previous tile's
     // reads, these stores, this tile's reads
@@ -229,7 +240,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) __attribute__((amdgpu_waves_per_eu
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
       const int c = lane + 64 * i;
-      *reinterpret_cast<u32x4*>(kl + (c / CPR) * KP + (c % CPR) * V) = kreg[i];
+      *reinterpret_cast<u32x4*>(kl + k_at(c / CPR, c % CPR)) = kreg[i];
       *reinterpret_cast<u32x4*>(vl + (c / CPR) * VRP + (c % CPR) * V) = vreg[i];
     }
     asm volatile("" ::: "memory");
@@ -239,7 +250,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) __attribute__((amdgpu_waves_per_eu
     for (int r = 0; r < 16; ++r) s[r] = 0.f;
 #pragma unroll
     for (int k = 0; k < NDS; ++k)
-      s = rows_mfma(*reinterpret_cast<const u32x4*>(kl + krow * KP + 16 * k + hf * V), qf[k], s);
+      s = rows_mfma(*reinterpret_cast<const u32x4*>(kl + k_at(krow, 2 * k + hf)), q_lds[k][lane], s);
     const int k0 = kbeg + t * kRowsKeys;
     if (k0 + kRowsKeys > minlen) {  // some row's last key lies in or before this tile (uniform)
 #pragma unroll
@@ -262,42 +273,42 @@ __global__ __launch_bounds__(64 * kRowsWaves) __attribute__((amdgpu_waves_per_eu
     ls += __shfl_xor(ls, 32, 64);
     lrun = fmaf(lrun, corr, ls);
     mrun = mnew;
+    if (__builtin_amdgcn_ballot_w64(corr != 1.f)) {
+#pragma unroll
+      for (int db = 0; db < NDB; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[db][r] *= corr;
+    }
     if (special) {
-      if (__builtin_amdgcn_ballot_w64(corr != 1.f)) {
-#pragma unroll
-        for (int db = 0; db < NDB; ++db)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) o[db][r] *= corr;
-      }
-      // P through the K tile's LDS (its reads are done), then one key at a time
+      // P through the K tile's LDS (its reads are done), one key at a time, then
+      // zeros in V's place for the products below
       float* const pl32 = reinterpret_cast<float*>(kl);
       asm volatile("" ::: "memory");
 #pragma unroll
       for (int r = 0; r < 16; ++r) pl32[(16 * (r >> 3) + 8 * hf + (r & 7)) * 32 + col] = s[r];
       asm volatile("" ::: "memory");
       for (int key = 0; key < kRowsKeys && k0 + key < maxlen; ++key) {
-        if (k0 + key < lim) {
-          const float p = pl32[key * 32 + col];
+        const bool mine = k0 + key < lim;
+        const float p = mine ? pl32[key * 32 + col] : 0.f;
 #pragma unroll
-          for (int i = 0; i < 4 * NDB; ++i) {
-            const uint2 w = *reinterpret_cast<const uint2*>(vl + key * VRP + 8 * i + 4 * hf);
-            f32x16& oo = o[i >> 2];
-            const int b = 4 * (i & 3);
-            oo[b + 0] = fmaf(p, bf16_bits_to_f32(w.x & 0xffffu), oo[b + 0]);
-            oo[b + 1] = fmaf(p, bf16_bits_to_f32(w.x >> 16), oo[b + 1]);
-            oo[b + 2] = fmaf(p, bf16_bits_to_f32(w.y & 0xffffu), oo[b + 2]);
-            oo[b + 3] = fmaf(p, bf16_bits_to_f32(w.y >> 16), oo[b + 3]);
-            __builtin_amdgcn_sched_barrier(0);
-          }
+        for (int i = 0; i < 4 * NDB; ++i) {
+          const uint2 w = *reinterpret_cast<const uint2*>(vl + key * VRP + 8 * i + 4 * hf);
+          f32x16& oo = o[i >> 2];
+          const int b = 4 * (i & 3);
+          oo[b + 0] = fmaf(p, mine ? bf16_bits_to_f32(w.x & 0xffffu) : 0.f, oo[b + 0]);
+          oo[b + 1] = fmaf(p, mine ? bf16_bits_to_f32(w.x >> 16) : 0.f, oo[b + 1]);
+          oo[b + 2] = fmaf(p, mine ? bf16_bits_to_f32(w.y & 0xffffu) : 0.f, oo[b + 2]);
+          oo[b + 3] = fmaf(p, mine ? bf16_bits_to_f32(w.y >> 16) : 0.f, oo[b + 3]);
+          __builtin_amdgcn_sched_barrier(0);
         }
       }
-      continue;
-    }
-    if (__builtin_amdgcn_ballot_w64(corr != 1.f)) {
+      asm volatile("" ::: "memory");
 #pragma unroll
-      for (int db = 0; db < NDB; ++db)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) o[db][r] *= corr;
+      for (int i = 0; i < NCH; ++i) {
+        const int c = lane + 64 * i;
+        *reinterpret_cast<u32x4*>(vl + (c / CPR) * VRP + (c % CPR) * V) = zero16();
+      }
+      asm volatile("" ::: "memory");
     }
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
