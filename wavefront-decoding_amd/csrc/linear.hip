@@ -45,8 +45,8 @@
 //  * block (bf16; n > 16 with more than 512 tiles, n > 32 with more than 256,
 //    else n > 256 and work enough): 64 or 128 rows x 64 or 128 columns per workgroup, half-chunk
 //    stages through an LDS ring.
-//  * gemm, slice form (wfd_linear_partials): the gemm kernel over one slice
-//    of K per workgroup (grid y = slice), storing fp32 slice partials.
+//  * gemm and block, slice forms (wfd_linear_partials): one slice of K per
+//    workgroup (grid y = slice), storing fp32 slice partials.
 //
 // So y[m] is bit-identical whatever n is and wherever row m sits -- the
 // property that keeps wavefront decode token-identical to sequential decode.
@@ -1167,6 +1167,9 @@ __global__ __launch_bounds__(256) void linear_stream_kernel(const T* __restrict_
 // dot products, so the same bits): a lane ends with 4 consecutive columns of
 // one row, which it stores at once, a RoPE pair in its own registers.
 //
+// PART (the slice form behind wfd_linear_partials, as the gemm's): grid y =
+// slice, the workgroup walks its slice's chunks and stores the slice sums.
+//
 // ONE: one chunk per sub-slice (K of at most 16 chunks): the chunk partial is
 // the sub-slice sum ((0 + c) added to a sum that is never -0 leaves the bits of
 // c added to it), so no sub-slice registers.
@@ -1226,10 +1229,11 @@ __device__ __forceinline__ void store_out4(TO* __restrict__ y, int64_t ldy, cons
   }
 }
 
-template <typename T, typename TO, int EPI, int NW, int RW, int CT, int NS, bool ONE>
+template <typename T, typename TO, int EPI, int NW, int RW, int CT, int NS, bool ONE, bool PART>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW / 4))) void linear_block_kernel(
     const T* __restrict__ x, const int32_t* __restrict__ x_rows, int64_t ldx, const T* __restrict__ W,
-    TO* __restrict__ y, int64_t ldy, int n, int K, int tiles, const RopeArgs ra, const float* __restrict__ rscale) {
+    TO* __restrict__ y, int64_t ldy, int n, int K, int tiles, const RopeArgs ra, float* __restrict__ part,
+    const float* __restrict__ rscale) {
   constexpr int V = LinTraits<T>::V;
   constexpr int KH = LinTraits<T>::KC / 2;  // elements per half chunk
   constexpr int CW = NW / RW;      // column groups
@@ -1257,21 +1261,24 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW / 4)
   const int row0 = rbk * BR + 32 * rw;
   const bool rows = row0 < n;  // uniform over the wave
   const int P = K / LinTraits<T>::KC;
+  // chunks [pb, pb + PN): all of K, or (PART) the slice of this workgroup
+  const int pb = PART ? (int)blockIdx.y * slice_chunks(P) : 0;
+  const int PN = PART ? min(P - pb, slice_chunks(P)) : P;
 
   const T* wsrc[WPW];
 #pragma unroll
   for (int i = 0; i < WPW; ++i) {
     const int f = wave * WPW + i;  // (tile f / 2, step f % 2 of the half)
     const int g = tg * BT + f / 2;
-    wsrc[i] = W + packed_off<T>(g < tiles ? g : tiles - 1, 0, P, lane) + (int64_t)(f % 2) * 64 * V;
+    wsrc[i] = W + packed_off<T>(g < tiles ? g : tiles - 1, pb, P, lane) + (int64_t)(f % 2) * 64 * V;
   }
   const T* xsrc[XPW];
 #pragma unroll
   for (int i = 0; i < XPW; ++i) {
     const int r = 8 * (wave * XPW + i) + (lane >> 3);
-    xsrc[i] = half_x_ptr<T>(x, x_rows, ldx, rbk * BR + r, (lane & 7) ^ ((r >> 1) & 7), n);
+    xsrc[i] = half_x_ptr<T>(x, x_rows, ldx, rbk * BR + r, (lane & 7) ^ ((r >> 1) & 7), n) + (int64_t)pb * LinTraits<T>::KC;
   }
-  const int H2 = 2 * P;  // half chunks; half h: steps 2 (h % 2), 2 (h % 2) + 1 of chunk h / 2
+  const int H2 = 2 * PN;  // half chunks; half h: steps 2 (h % 2), 2 (h % 2) + 1 of chunk pb + h / 2
   auto issue = [&](int h) {
     const int st = h % NS;
 #pragma unroll
@@ -1283,7 +1290,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW / 4)
   for (int u = 0; u < NS - 1; ++u)
     if (u < H2) issue(u);
 
-  SliceWalk walk(P, 0);
+  SliceWalk walk(P, pb);
   f32x4 sub[2][CT], sl[2][CT], tot[2][CT];
   f32x4 acc0[2][CT], acc1[2][CT];  // chunk partials: even chunks, odd chunks
 #pragma unroll
@@ -1329,7 +1336,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW / 4)
       }
   };
   auto close = [&](int p) {
-    const int lvl = walk.end(p);
+    const int lvl = walk.end(pb + p);
     if (!ONE && lvl >= 1) into(sl, sub);
     if (lvl == 2) into(tot, sl);
   };
@@ -1378,21 +1385,30 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW / 4)
     wait_vmem_barrier<0>();
   read(xa, wa, 0, 0);
   int p = 0;
-  for (; p + 1 < P; p += 2) {
+  for (; p + 1 < PN; p += 2) {
     chunk(acc0, acc1, p);  // before chunk 0: adds zeros
     chunk(acc1, acc0, p + 1);
   }
-  if (p < P) {
+  if (p < PN) {
     chunk(acc0, acc1, p);
     add(acc0);
   } else {
     add(acc1);
   }
-  close(P - 1);
+  close(PN - 1);
   if (!rows) return;  // after the last barrier; every load of this wave has completed
 #pragma unroll
   for (int a = 0; a < 2; ++a) {
     const int row = row0 + 16 * a + (lane & 15);
+    if constexpr (PART) {  // the slice sums
+#pragma unroll
+      for (int t = 0; t < CT; ++t) {
+        const int g = tg * BT + cw * CT + t;
+        if (g < tiles && row < n)
+          *reinterpret_cast<f32x4*>(part + ((int64_t)blockIdx.y * n + row) * 16 * tiles + 16 * g + 4 * grp) = tot[a][t];
+      }
+      continue;
+    }
     const int rc = row < n ? row : n - 1;
     const float sc = rscale ? rscale[rc] : 1.f;  // a folded norm pair's row scale
     int pos = 0;
@@ -1448,24 +1464,25 @@ static WidePlan wide_plan(int n, int tiles, int R, bool swiglu) {
 // lm_head are faster here: 16.5 -> 14.7, 30.5 -> 25.3 us).
 enum BlockShape : int { kBlockNone = 0, kBlock128x128, kBlock128x64, kBlock64x64 };
 
-static int block_shape(int n, int tiles) {
+static int block_shape(int n, int tiles, int S) {
   const long rb128 = (n + 127) / 128, rb64 = (n + 63) / 64, g8 = (tiles + 7) / 8, g4 = (tiles + 3) / 4;
-  if ((tiles <= kStreamMaxTiles && (n <= 256 || rb64 * g4 < 160)) || (tiles <= kGemmMinBlockTiles && n <= 32))
+  if (S == 1 && ((tiles <= kStreamMaxTiles && (n <= 256 || rb64 * g4 < 160)) || (tiles <= kGemmMinBlockTiles && n <= 32)))
     return kBlockNone;
-  const long a = 37 * ((rb128 * g8 + 255) / 256);
-  const long b = 27 * ((rb128 * g4 + 255) / 256);
-  const long c = rb64 * g4 <= 256 ? 23 : 34 * ((rb64 * g4 + 511) / 512);
+  const long a = 37 * ((rb128 * g8 * S + 255) / 256);
+  const long b = 27 * ((rb128 * g4 * S + 255) / 256);
+  const long c = rb64 * g4 * S <= 256 ? 23 : 34 * ((rb64 * g4 * S + 511) / 512);
   return a <= b && a <= c ? kBlock128x128 : b <= c ? kBlock128x64 : kBlock64x64;
 }
 
-template <typename TO, int EPI>
+template <typename TO, int EPI, bool PART>
 static void launch_block(int shape, const void* x, const int32_t* xr, int64_t ldx, const void* W, void* y, int64_t ldy,
-                         int n, int K, int tiles, bool one, const RopeArgs& ra, const float* rsc, hipStream_t st) {
+                         int n, int K, int tiles, bool one, int S, const RopeArgs& ra,
+                         float* part, const float* rsc, hipStream_t st) {
 #define WFD_BLOCK(NW, RW, CT, ONE)                                                                              \
-  hipLaunchKernelGGL((linear_block_kernel<bf16_t, TO, EPI, NW, RW, CT, 4, ONE>),                               \
-                     dim3(xcd_grid((n + 32 * RW - 1) / (32 * RW), (tiles + NW / RW * CT - 1) / (NW / RW * CT))), \
+  hipLaunchKernelGGL((linear_block_kernel<bf16_t, TO, EPI, NW, RW, CT, 4, ONE, PART>),                               \
+                     dim3(xcd_grid((n + 32 * RW - 1) / (32 * RW), (tiles + NW / RW * CT - 1) / (NW / RW * CT)), S), \
                      dim3(64 * NW), 0, st, (const bf16_t*)x, xr, ldx, (const bf16_t*)W, (TO*)y, ldy, n, K, tiles, \
-                     ra, rsc)
+                     ra, part, rsc)
   if (shape == kBlock128x128) {
     if (one) WFD_BLOCK(16, 4, 2, true);
     else WFD_BLOCK(16, 4, 2, false);
@@ -1513,9 +1530,9 @@ static void launch_linear(const void* x, const int32_t* xr, int64_t ldx, const v
     const float* rsc = rs.scale;  // many rows: the scales precomputed (group sums are few-row only)
     const int rb = (n + 63) / 64;
     if constexpr (std::is_same<T, bf16_t>::value) {
-      const int bs = block_shape(n, tiles);
+      const int bs = block_shape(n, tiles, 1);
       if (bs != kBlockNone) {
-        launch_block<TO, EPI>(bs, x, xr, ldx, W, y, ldy, n, K, tiles, R == 1, ra, rsc, st);
+        launch_block<TO, EPI, false>(bs, x, xr, ldx, W, y, ldy, n, K, tiles, R == 1, 1, ra, nullptr, rsc, st);
         return;
       }
     }
@@ -1569,6 +1586,15 @@ static void launch_linear_partials(const void* x, const int32_t* xr, int64_t ldx
   const int S = slice_count(P);
   const int rb = (n + 63) / 64;
   const RopeArgs ra{};
+  // the block kernel's slice form: 2048 columns x 2048 / 4096 / 5632 inputs at 64 /
+  // 128 / 256 / 512 rows 5.7 / 6.7 / 9.5 / 14.4, 8.4 / 9.9 / 14.2 / 24.2 and 10.7 / 11.4 / 16.8 / 28.5
+  // us with the 64-row gemm workgroups, 5.2 / 5.5 / 7.3 / 10.8, 9.3 / 9.4 / 12.8 / 17.4 and
+  // 11.9 / 11.7 / 16.1 / 21.7 with it: longer slices of few rows stay on the gemm
+  if (std::is_same<T, bf16_t>::value && (n > 96 || sub_chunks(P) == 1)) {
+    launch_block<bf16_t, kEpiPlain, true>(block_shape(n, tiles, S), x, xr, ldx, W, nullptr, 0, n, K, tiles,
+                                          sub_chunks(P) == 1, S, ra, part, nullptr, st);
+    return;
+  }
   const int bt = gemm_tiles_per_workgroup(rb, tiles, S);
 #define WFD_GEMM_PART(BTV)                                                                                          \
   hipLaunchKernelGGL((linear_gemm_kernel<T, T, kEpiPlain, BTV, true>), dim3(xcd_grid(rb, (tiles + BTV - 1) / BTV), S), \
