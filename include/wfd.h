@@ -305,7 +305,7 @@ int wfd_linear_prep(const void* x, const int32_t* x_rows, int64_t ldx, const voi
                     const wfd_prep_t* pp, wfd_stream_t stream);
 
 /*
- * The row form of a folded norm pair, one wave per row: the row y is
+ * The row form of a folded norm pair: the row y is
  * a[i * lda] (part NULL) or the in-order slice sum of wfd_linear_partials'
  * part (rounded to dtype, wfd_linear's output bit for bit); r and A as
  * wfd_linear_prep computes them (r into pp->r_out if given), scale_out[i] =
@@ -329,8 +329,8 @@ int wfd_norm_prep(const void* a, int64_t lda, const float* part, int64_t slice_s
 int wfd_linear_slices(int K, int dtype);
 
 /*
- * Split-K form of wfd_linear (plain epilogue): one workgroup per (64 rows,
- * 32 or 64 columns, K slice), so a many-row projection with few output
+ * Split-K form of wfd_linear (plain epilogue): one workgroup per (64 or 128 rows,
+ * 32 to 128 columns, K slice), so a many-row projection with few output
  * columns fills the chip and reads each x row once per 32-64 columns. Writes
  * the fp32 slice sums part[(q * n + m) * N + j] for q < wfd_linear_slices(K);
  * adding them in slice order from zero and rounding to dtype gives wfd_linear's
