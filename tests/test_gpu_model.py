@@ -103,6 +103,30 @@ def test_prompt_pass_library_gemm_matches_kernels(gpu, dtype):
         assert rel_err(outs[0][0], ref) <= tol
 
 
+@pytest.mark.parametrize("L", [128, 129, 257, 641])
+def test_prompt_pass_mixes_packed_and_library_linears(gpu, L):
+    """bf16 prompts on both sides of the row counts up to which each linear of
+    the pass stays on the packed kernels (down 128, gate|up and the adapter 256,
+    q|k|v and proj 640): the slot caches and the logits agree with the pass that
+    never leaves them, to the tolerance of the two GEMM orders' roundings."""
+    import dataclasses
+    cfg = dataclasses.replace(TINY, dtype="bfloat16")
+    w = M.init_weights(cfg, 0)
+    ids = _prompt(L).tolist()
+    outs = []
+    for dense in (True, False):
+        m = LoopedModel(cfg, w, gpu, max_seq_len=L + 3, max_batch=1, dense_prompt=dense)
+        assert dense is False or [m._library_rows(k, L) for k in ("mlp_proj", "fc", "Wqkv")] == [L > 128, L > 256,
+                                                                                                 L > 640]
+        cache = m.create_cache(1)
+        logits = m.prefill_seq(cache, 0, ids)
+        torch.cuda.synchronize()
+        outs.append((logits.float().cpu().numpy(), cache.flat_k.float().cpu().numpy(),
+                     cache.flat_v.float().cpu().numpy()))
+    for a, b in zip(outs[0], outs[1]):
+        assert rel_err(a, b) <= 5e-2
+
+
 @pytest.mark.parametrize("T_draft", [1, 2])
 def test_tiny_wfd_matches_oracle_and_sequential(tiny, T_draft):
     w, model = tiny

@@ -1458,7 +1458,8 @@ static WidePlan wide_plan(int n, int tiles, int R, bool swiglu) {
 // 17 for up to 512; the shape with the fewest rounds by that measure was the
 // fastest, or within 3 %, at 64-1500 rows x 128-2000 tiles. With at most
 // kStreamMaxTiles tiles the stream kernel's one- and two-tile workgroups fill
-// more CUs up to 256 rows and below 160 of the 64 x 64 workgroups (2048 x 5632 at 64 / 192 / 512 rows: stream 18 / 24 / 46,
+// more CUs up to 256 rows, below 160 of the 64 x 64 workgroups or below their 4
+// tiles (2048 x 5632 at 64 / 192 / 512 rows: stream 18 / 24 / 46,
 // block 30 / 30 / 31 us); at 32 rows or fewer and up to 512 tiles the tile kernel
 // streams the weights without barriers (q|k|v 11.7 against 12.4 us; gate|up and
 // lm_head are faster here: 16.5 -> 14.7, 30.5 -> 25.3 us).
@@ -1466,7 +1467,7 @@ enum BlockShape : int { kBlockNone = 0, kBlock128x128, kBlock128x64, kBlock64x64
 
 static int block_shape(int n, int tiles, int S) {
   const long rb128 = (n + 127) / 128, rb64 = (n + 63) / 64, g8 = (tiles + 7) / 8, g4 = (tiles + 3) / 4;
-  if (S == 1 && ((tiles <= kStreamMaxTiles && (n <= 256 || rb64 * g4 < 160)) || (tiles <= kGemmMinBlockTiles && n <= 32)))
+  if (S == 1 && ((tiles <= kStreamMaxTiles && (n <= 256 || tiles < 4 || rb64 * g4 < 160)) || (tiles <= kGemmMinBlockTiles && n <= 32)))
     return kBlockNone;
   const long a = 37 * ((rb128 * g8 * S + 255) / 256);
   const long b = 27 * ((rb128 * g4 * S + 255) / 256);
