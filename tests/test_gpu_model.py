@@ -116,8 +116,8 @@ def test_prompt_pass_mixes_packed_and_library_linears(gpu, L):
     outs = []
     for dense in (True, False):
         m = LoopedModel(cfg, w, gpu, max_seq_len=L + 3, max_batch=1, dense_prompt=dense)
-        assert dense is False or [m._library_rows(k, L) for k in ("mlp_proj", "fc", "Wqkv")] == [L > 128, L > 256,
-                                                                                                 L > 640]
+        assert m._library_linears(L) == {k for k, r in (("mlp_proj", 128), ("fc", 256), ("adapter", 256), ("Wqkv", 640),
+                                                        ("proj", 640)) if dense and L > r}
         cache = m.create_cache(1)
         logits = m.prefill_seq(cache, 0, ids)
         torch.cuda.synchronize()

@@ -368,19 +368,18 @@ class LoopedModel:
     # -- one SandwichBlock over n rows --------------------------------------------
     def _block(self, prefix: str, n: int, sc, pos_d, kvlen_d, rb_d, fr_d, kv_len_max: int, ws,
                cache: BatchStaticKVCache, next_norm: torch.Tensor | None, final_out=None, final_rows=None,
-               segments=None, group_first=None, dense: bool = False):
+               segments=None, group_first=None, library: frozenset = frozenset()):
         """One SandwichBlock over n rows. `segments` = (seg_row_base, seg_q_start,
         seg_pos0, max_seg_len) routes attention through the causal prefill
         kernel (rows grouped by slot at consecutive positions) instead of the
         per-row decode kernel; `group_first` groups decode rows that share a
-        slot (one prefix read per group, same bits). `dense` (the prompt pass)
-        runs the linears beyond the packed kernels' row range (_library_rows) as
-        library GEMMs over the row-major weights, with the RoPE/append and
+        slot (one prefix read per group, same bits). `library` names the linears
+        that the prompt pass runs (beyond the packed kernels' row range) as library
+        GEMMs over the row-major weights, with the RoPE/append and
         SwiGLU epilogues as their own kernels."""
         c, W = self.cfg, self.W
         x, h = sc["x"], sc["h"]
-        lib = lambda leaf: dense and self._library_rows(leaf, n)  # noqa: E731
-        if lib("Wqkv"):
+        if "Wqkv" in library:
             qkv = torch.mm(h[:n], self.Wd[prefix + "Wqkv"].t(), out=sc["qkv"][:n])
             q = ops.qkv_rope_append(qkv, pos_d, self.rope_cos, self.rope_sin, fr_d, cache.flat_k, cache.flat_v,
                                     c.n_heads, c.n_kv_heads, c.head_dim, q_out=sc["q"][:n])
@@ -394,30 +393,31 @@ class LoopedModel:
         else:
             o = ops.attn_decode(q, cache.flat_k, cache.flat_v, rb_d, kvlen_d, kv_len_max=kv_len_max,
                                 out=sc["o"][:n], workspace=ws, group_first=group_first)
-        if lib("proj"):
+        if "proj" in library:
             a = torch.mm(o.view(n, -1), self.Wd[prefix + "proj"].t(), out=sc["a"][:n])
             ops.add_rmsnorm(a, W[prefix + "norm_2"], c.norm_eps, res=x, w2=W[prefix + "norm_3"], n=n, x_out=x,
                             h_out=h)
         else:
             self._linear_norm(o.view(n, -1), W[prefix + "proj"], n, sc, "a", W[prefix + "norm_2"], res=x,
                               w2=W[prefix + "norm_3"], x_out=x, h_out=h)
-        if lib("fc"):
+        if "fc" in library:
             gu = torch.mm(h[:n], self.Wd[prefix + "fc"].t(), out=sc["gu"][:n])
             u = ops.swiglu(gu, n=n, out=sc["u"][:n])
         else:
             u = ops.linear(h, W[prefix + "fc"], n=n, out=sc["u"], swiglu=True)
         out = (dict(w2=next_norm, x_out=x, h_out=h) if next_norm is not None
                else dict(x_out=final_out, out_rows=final_rows))
-        if lib("mlp_proj"):
+        if "mlp_proj" in library:
             m = torch.mm(u[:n], self.Wd[prefix + "mlp_proj"].t(), out=sc["m"][:n])
             ops.add_rmsnorm(m, W[prefix + "norm_4"], c.norm_eps, res=x, n=n, **out)
         else:
             self._linear_norm(u, W[prefix + "mlp_proj"], n, sc, "m", W[prefix + "norm_4"], res=x, **out)
 
-    def _library_rows(self, leaf: str, n: int) -> bool:
-        """Whether the prompt pass runs this linear over n rows as a library
-        GEMM (with dense_prompt): beyond the packed kernels' range (bf16), or fp32."""
-        return self.dtype != torch.bfloat16 or n > _PACKED_PROMPT_ROWS[leaf]
+    def _library_linears(self, n: int) -> frozenset:
+        """The linears that a prompt pass over n rows runs as library GEMMs: with
+        dense_prompt, those beyond the packed kernels' range (bf16), or all (fp32)."""
+        return frozenset(leaf for leaf, rows in _PACKED_PROMPT_ROWS.items()
+                         if self.dense_prompt and (self.dtype != torch.bfloat16 or n > rows))
 
     def _linear_norm(self, xin: torch.Tensor, Wp, n: int, sc, tmp: str, w1: torch.Tensor, *, x_rows=None,
                      keep=None, **norm) -> None:
@@ -836,7 +836,7 @@ class LoopedModel:
         """Whole prompt of sequence b at positions [0, L): fills every slot's
         [0, L) and returns the last position's logits (V,) float32. Runs eagerly
         with its own L-row scratch; with dense_prompt its larger linears are library
-        GEMMs (see __init__, _library_rows), the last position's lm_head row the packed kernel."""
+        GEMMs (see __init__, _library_linears), the last position's lm_head row the packed kernel."""
         c, W = self.cfg, self.W
         ids = np.asarray(token_ids, dtype=np.int64).reshape(-1)
         L = len(ids)
@@ -860,8 +860,8 @@ class LoopedModel:
         flash = self.dtype == torch.bfloat16 and c.head_dim in (64, 128)
         seg_l = (lambda s: (t64[2 * n_layers * L + s: 2 * n_layers * L + s + 1], t32[2 * L: 2 * L + 2],  # noqa: E731
                             t32[2 * L + 2: 2 * L + 3], L)) if flash else (lambda s: None)
-        dense = self.dense_prompt
-        sc = self._scratch(L, dense=dense)
+        library = self._library_linears(L)
+        sc = self._scratch(L, dense=bool(library))
         ws = None if flash else torch.zeros(ops.attn_workspace_bytes(L, c.n_heads, c.head_dim, L),
                                             dtype=torch.uint8, device=self.device)
         logits = torch.empty(1, c.vocab_size, dtype=torch.float32, device=self.device)
@@ -871,10 +871,10 @@ class LoopedModel:
         for i in range(c.n_prelude):
             nxt = W[f"prelude.{i + 1}.norm_1"] if i + 1 < c.n_prelude else None
             self._block(f"prelude.{i}.", L, sc, pos_d, kvlen_d, rb_l(i), fr_l(i), L, ws, cache, nxt,
-                        final_out=state[:, D:], segments=seg_l(i), dense=dense)
+                        final_out=state[:, D:], segments=seg_l(i), library=library)
         state[:, :D].copy_(self._prompt_s0(L))
         for r in range(c.T_total):
-            if dense and self._library_rows("adapter", L):
+            if "adapter" in library:
                 torch.mm(state, self.Wd["adapter"].t(), out=sc["x"][:L])
             else:
                 ops.linear(state, W["adapter"], n=L, out=sc["x"])
@@ -883,13 +883,13 @@ class LoopedModel:
                 s = self.slot_core(r, l)
                 nxt = W[f"core.{l + 1}.norm_1"] if l + 1 < c.n_core else None
                 self._block(f"core.{l}.", L, sc, pos_d, kvlen_d, rb_l(s), fr_l(s), L, ws, cache, nxt,
-                            final_out=state[:, :D], segments=seg_l(s), dense=dense)
+                            final_out=state[:, :D], segments=seg_l(s), library=library)
         ops.add_rmsnorm(state, W["ln_f"], c.norm_eps, w2=W["coda.0.norm_1"], n=L, x_out=sc["x"], h_out=sc["h"])
         for i in range(c.n_coda):
             s = self.slot_coda(i)
             nxt = W[f"coda.{i + 1}.norm_1"] if i + 1 < c.n_coda else W["ln_f"]
             self._block(f"coda.{i}.", L, sc, pos_d, kvlen_d, rb_l(s), fr_l(s), L, ws, cache, nxt, segments=seg_l(s),
-                        dense=dense)
+                        library=library)
         ops.linear(sc["h"][L - 1: L], W["lm_head"], n=1, out=logits, out_dtype=torch.float32)
         for s in range(n_layers):
             cache.seqlen[s][b] = max(cache.seqlen[s][b], L)
