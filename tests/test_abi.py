@@ -85,6 +85,26 @@ def test_host_only_entry_points():
     assert lib.wfd_linear_pack(8, 16, 32, 128, 1, 1, 12, None) == -1     # swiglu pair_off mismatch
 
 
+def test_varlen_entry_point_checks_before_launch():
+    """wfd_attn_varlen refuses bad shapes, types, scales and pointers on the
+    host, and its workspace holds the row tables (8 + 4 bytes a row), the tile
+    table (a tile per 32 / G rows and one more per segment) and, past one key
+    split, the split partials."""
+    lib = _lib.load()
+    call = lambda *a: lib.wfd_attn_varlen(None, None, None, None, None, None, *a, None, 0, None)  # noqa: E731
+    assert call(1, 4, 16, 3, 128, 1, 0.1, 10, 1) == -1 and b"bad shape" in lib.wfd_last_error()
+    assert call(1, 4, 16, 16, 128, 1, 0.1, 0, 1) == -1 and b"max_k=0" in lib.wfd_last_error()
+    assert call(1, 4, 16, 16, 128, 1, 0.0, 10, 1) == -1 and b"positive" in lib.wfd_last_error()
+    assert call(1, 4, 16, 16, 128, 0, 0.1, 10, 1) == -2 and call(1, 4, 16, 16, 96, 1, 0.1, 10, 1) == -2
+    assert call(1, 4, 16, 2, 128, 1, 0.1, 10, 1) == -2 and b"G=8" in lib.wfd_last_error()
+    assert call(1, 0, 16, 16, 128, 1, 0.1, 10, 1) == 0
+    assert call(1, 4, 16, 16, 128, 1, 0.1, 10, 1) == -1 and b"null pointer" in lib.wfd_last_error()
+    tables = lambda n, tiles: sum(-(-b // 256) * 256 for b in (8 * n, 4 * n, 4 * tiles))  # noqa: E731
+    assert lib.wfd_attn_varlen_workspace_bytes(5, 100, 16, 16, 128, 1024) == tables(100, 100 // 32 + 5 + 3)
+    assert (lib.wfd_attn_varlen_workspace_bytes(5, 100, 16, 4, 128, 1025)
+            == tables(100, 100 // 8 + 5 + 3) + lib.wfd_attn_workspace_bytes(100, 16, 128, 1025))
+
+
 @pytest.mark.skipif(torch.cuda.device_count() > 0, reason="made-up device addresses: run only where no GPU is "
                     "visible, so a regressed check cannot launch a kernel on them")
 def test_alignment_and_grid_checks_reject_before_launch():

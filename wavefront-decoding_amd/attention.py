@@ -80,6 +80,10 @@ def _cached(key, build):
     return t
 
 
+def _raw_stream(device: torch.device) -> int:
+    return torch._C._cuda_getCurrentRawStream(device.index)
+
+
 def _scale(Dh: int) -> float:
     return 1.0 / math.sqrt(Dh)
 
@@ -126,7 +130,7 @@ def _dense_offsets(B: int, Tq: int, Tk: int, device):
         s = torch.arange(B + 1, dtype=torch.int32)
         return (s * Tq).to(device), (s * Tk).to(device)
 
-    return _cached(("dense_cu", B, Tq, Tk, str(device)), build)
+    return _cached(("dense_cu", B, Tq, Tk, device, _raw_stream(device)), build)
 
 
 def attn_dense(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, causal: bool) -> torch.Tensor:
@@ -226,12 +230,13 @@ def _fused_qkv_weight(attn):
 
 def _token_tables(B: int, T: int, device):
     """(positions 0..T-1 of every batch row, int32; row numbers, int64) of B * T
-    packed tokens. One pair per shape, built on the host and copied; a stream
-    under capture gets its own, which the graph then owns."""
+    packed tokens. One pair per shape and stream (a pair that the table drops is
+    reused in the order of the stream that reads it), built on the host and
+    copied; a stream under capture gets its own, which the graph then owns."""
     if torch.cuda.is_current_stream_capturing():
         return (torch.arange(T, dtype=torch.int32, device=device).repeat(B),
                 torch.arange(B * T, dtype=torch.int64, device=device))
-    return _cached(("tokens", B, T, str(device)), lambda: (torch.arange(T, dtype=torch.int32).repeat(B).to(device),
+    return _cached(("tokens", B, T, device, _raw_stream(device)), lambda: (torch.arange(T, dtype=torch.int32).repeat(B).to(device),
                                                            torch.arange(B * T, dtype=torch.int64).to(device)))
 
 
