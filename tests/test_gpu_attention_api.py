@@ -299,3 +299,61 @@ def test_compute_qkv_reference_form(gpu, dtype, H, Hkv, Dh):
         attn.c_k.weight.mul_(-1)  # in place: the packed copy must be rebuilt
     q4, k4, v4 = A.compute_qkv(attn, x, freqs)
     assert torch.equal(q4, q) and torch.equal(v4, v) and torch.equal(k4, -k)
+
+
+def _capture(fn):
+    """fn() as a graph, captured on torch's own capture stream after one call
+    on the current one: (graph, the outputs it writes)."""
+    fn()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = fn()
+    torch.cuda.synchronize()
+    return graph, out if isinstance(out, tuple) else (out,)
+
+
+@pytest.mark.parametrize("form", ["prompt", "whole", "short keys", "one row", "fp32 rows", "q1", "qkv"])
+def test_captured_calls_replay_after_other_shapes(gpu, form):
+    """Each entry point that uses index tables, captured after a warm-up on
+    another stream, then replayed on new inputs after 300 other shapes have
+    gone through the module (more than it keeps) and their memory has been
+    reused: the eager call's bits every time."""
+    H, Hkv, Dh, B = 4, 4, 64, 2
+    Tq, Tk = {"prompt": (70, 90), "whole": (90, 70), "short keys": (90, 70), "one row": (1, 70),
+              "fp32 rows": (5, 70)}.get(form, (1, 1))
+    dt = torch.float32 if form == "fp32 rows" else torch.bfloat16
+    g = torch.Generator().manual_seed(len(form))
+    mk = lambda *s: torch.randn(*s, generator=g).to(dt).to(gpu)  # noqa: E731
+    if form == "qkv":
+        attn = type("Attn", (), dict(Wqkv=ops.pack_linear(0.05 * mk((H + 2 * Hkv) * Dh, 256)), n_head=H,
+                                     n_kv_head=Hkv, head_dim=Dh))
+        ang = torch.rand(33, Dh // 2, generator=g)
+        freqs = torch.polar(torch.ones_like(ang), ang).to(gpu)
+        ins = [mk(B, 33, 256)]
+        fn = lambda: A.compute_qkv(attn, ins[0], freqs)  # noqa: E731
+    elif form == "q1":
+        cu = torch.tensor([0, 40, 41, 200], dtype=torch.int32, device=gpu)
+        ins = [mk(3, H, Dh), mk(200, Hkv, Dh), mk(200, Hkv, Dh)]
+        fn = lambda: A.attn_varlen_q1_padded(*ins, cu, 159)  # noqa: E731
+    else:
+        ins = [mk(B, Tq, H, Dh), mk(B, Tk, Hkv, Dh), mk(B, Tk, Hkv, Dh)]
+        fn = lambda: A.attn_dense(*ins, causal=form != "whole")  # noqa: E731
+    print(f"[captured {form}]", flush=True)
+    graph, outs = _capture(fn)
+    x = torch.zeros(1, 400, 256, dtype=torch.bfloat16, device=gpu)
+    small = type("Small", (), dict(Wqkv=ops.pack_linear(torch.zeros(48, 256, dtype=torch.bfloat16, device=gpu)),
+                                   n_head=1, n_kv_head=1, head_dim=16))
+    ones = torch.ones(400, 8, dtype=torch.complex64, device=gpu)
+    for T in range(1, 301):
+        A.compute_qkv(small, x[:, :T], ones[:T])
+    junk = [torch.full((2048,), 0x7f7f7f7f, dtype=torch.int32, device=gpu) for _ in range(600)]
+    for _ in range(3):
+        for t in ins:
+            t.copy_(mk(*t.shape))
+        graph.replay()
+        torch.cuda.synchronize()
+        want = fn()
+        for a, b in zip(outs, want if isinstance(want, tuple) else (want,), strict=True):
+            assert torch.equal(a, b)
+    assert len(junk) == 600

@@ -72,6 +72,11 @@ _TABLES: dict[tuple, tuple[torch.Tensor, ...]] = {}
 
 
 def _cached(key, build):
+    """The tables `build` makes on the device, kept by `key`. A stream under
+    capture gets tables of its own: built inside the capture, so that the
+    graph owns their memory and replays never read a table dropped since."""
+    if torch.cuda.is_current_stream_capturing():
+        return build()
     t = _TABLES.get(key)
     if t is None:
         if len(_TABLES) > 256:
@@ -90,20 +95,20 @@ def _scale(Dh: int) -> float:
 
 def _dense_rows(B: int, Tq: int, Tk: int, causal: bool, device) -> tuple[torch.Tensor, torch.Tensor]:
     def build():
-        b = torch.arange(B, dtype=torch.int64).repeat_interleave(Tq)
-        j = torch.arange(Tq, dtype=torch.int64).repeat(B)
-        kv = (Tk - Tq + j + 1).clamp(min=0) if causal else torch.full_like(j, Tk)
-        return (b * Tk).to(device), kv.to(torch.int32).to(device)
+        base = torch.arange(B, dtype=torch.int64, device=device).mul_(Tk).view(B, 1).expand(B, Tq).reshape(-1)
+        if not causal:
+            return base, torch.full((B * Tq,), Tk, dtype=torch.int32, device=device)
+        kv = torch.arange(Tk - Tq + 1, Tk + 1, dtype=torch.int32, device=device).clamp_(min=0)
+        return base, kv.expand(B, Tq).reshape(-1)
 
     return _cached(("dense", B, Tq, Tk, causal, str(device)), build)
 
 
 def _prefill_segments(B: int, Tq: int, Tk: int, device):
     def build():
-        rb = torch.arange(B, dtype=torch.int64) * Tk
-        qs = (torch.arange(B + 1, dtype=torch.int32) * Tq)
-        p0 = torch.full((B,), Tk - Tq, dtype=torch.int32)
-        return rb.to(device), qs.to(device), p0.to(device)
+        return (torch.arange(B, dtype=torch.int64, device=device).mul_(Tk),
+                torch.arange(B + 1, dtype=torch.int32, device=device).mul_(Tq),
+                torch.full((B,), Tk - Tq, dtype=torch.int32, device=device))
 
     return _cached(("prefill", B, Tq, Tk, str(device)), build)
 
@@ -127,8 +132,8 @@ def _shared_rows(total_q: int, nseg: int, max_k: int, H: int, Hkv: int, Dh: int)
 
 def _dense_offsets(B: int, Tq: int, Tk: int, device):
     def build():
-        s = torch.arange(B + 1, dtype=torch.int32)
-        return (s * Tq).to(device), (s * Tk).to(device)
+        s = torch.arange(B + 1, dtype=torch.int32, device=device)
+        return s * Tq, s * Tk
 
     return _cached(("dense_cu", B, Tq, Tk, device, _raw_stream(device)), build)
 
@@ -141,6 +146,7 @@ def attn_dense(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, causal: boo
     Bk, Tk, Hkv, Dk = k.shape
     if (Bk, Dk) != (B, Dh) or v.shape != k.shape:
         raise _lib.WfdError(f"attn_dense: q {tuple(q.shape)} / k {tuple(k.shape)} / v {tuple(v.shape)} do not match")
+    ops._need_cuda(q, k, v)
     qf = q.contiguous().view(B * Tq, H, Dh)
     kf = k.contiguous().view(B * Tk, Hkv, Dh)
     vf = v.contiguous().view(B * Tk, Hkv, Dh)
@@ -202,7 +208,9 @@ def attn_varlen_q1_padded(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu_
     """n single-query segments: q (n, H, Dh), row i attends the whole segment
     [cu_k[i], cu_k[i+1]) -- the result of the reference's padded form."""
     n = q.shape[0]
-    cu_q = _cached(("q1", n, str(q.device)), lambda: (torch.arange(n + 1, dtype=torch.int32).to(q.device),))[0]
+    ops._need_cuda(q)
+    cu_q = _cached(("q1", n, str(q.device)),
+                   lambda: (torch.arange(n + 1, dtype=torch.int32, device=q.device),))[0]
     return attn_varlen(q, k, v, cu_q, cu_k, 1, max_k, causal=False)
 
 
@@ -231,13 +239,10 @@ def _fused_qkv_weight(attn):
 def _token_tables(B: int, T: int, device):
     """(positions 0..T-1 of every batch row, int32; row numbers, int64) of B * T
     packed tokens. One pair per shape and stream (a pair that the table drops is
-    reused in the order of the stream that reads it), built on the host and
-    copied; a stream under capture gets its own, which the graph then owns."""
-    if torch.cuda.is_current_stream_capturing():
-        return (torch.arange(T, dtype=torch.int32, device=device).repeat(B),
-                torch.arange(B * T, dtype=torch.int64, device=device))
-    return _cached(("tokens", B, T, device, _raw_stream(device)), lambda: (torch.arange(T, dtype=torch.int32).repeat(B).to(device),
-                                                           torch.arange(B * T, dtype=torch.int64).to(device)))
+    reused in the order of the stream that reads it)."""
+    return _cached(("tokens", B, T, device, _raw_stream(device)),
+                   lambda: (torch.arange(T, dtype=torch.int32, device=device).repeat(B),
+                            torch.arange(B * T, dtype=torch.int64, device=device)))
 
 
 def _rope_tables(freqs, B: int, T: int, Dh: int, device):
@@ -298,6 +303,7 @@ def compute_qkv(attn, x: torch.Tensor, freqs, ve=None, config=None):
         k = qkv[:, H * Dh: (H + Hkv) * Dh].view(B, T, Hkv, Dh)
         v = qkv[:, (H + Hkv) * Dh:].view(B, T, Hkv, Dh)
         return q, k, v
+    ops._need_cuda(x)
     cos, sin, pos = _rope_tables(freqs, B, T, Dh, x.device)
     kbuf = torch.empty(n, Hkv, Dh, dtype=x.dtype, device=x.device)
     vbuf = torch.empty_like(kbuf)
