@@ -66,15 +66,73 @@ def test_tables_under_capture_belong_to_the_graph(monkeypatch):
     stream, capturing = [7], [False]
     monkeypatch.setattr(A, "_raw_stream", lambda device: stream[0])
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing[0])
-    monkeypatch.setattr(A, "_TABLES", type(A._TABLES)())
+    monkeypatch.setattr(A, "_TABLES", A._TableCache())
     for name, (call, want) in _table_calls(torch.device("cpu")).items():
         kept = call()
         assert all(torch.equal(a, b) and a.dtype == b.dtype for a, b in zip(kept, want, strict=True)), name
         assert all(a is b for a, b in zip(call(), kept)), name
-        before = set(A._TABLES)
+        before = set(A._TABLES.held)
         for s in (7, 8):  # the warmed-up stream, and the one torch.cuda.graph captures on
             stream[0], capturing[0] = s, True
             own = call()
             assert all(torch.equal(a, b) and a.data_ptr() != c.data_ptr() for a, b, c in zip(own, want, kept)), name
-            assert set(A._TABLES) == before, name
+            assert set(A._TABLES.held) == before, name
         stream[0], capturing[0] = 7, False
+
+
+def test_tables_stay_with_their_stream_and_shape(monkeypatch):
+    """A table is handed to the stream that built it only, and other shapes --
+    of any entry point, on any stream -- push out the least recently used
+    tables one by one, never one in use; few or huge ones, within the bytes."""
+    stream = [7]
+    monkeypatch.setattr(A, "_raw_stream", lambda device: stream[0])
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(A, "_TABLES", A._TableCache())
+    dev = torch.device("cpu")
+    for name, (call, _) in _table_calls(dev).items():
+        mine = call()
+        stream[0] = 8
+        assert not {t.data_ptr() for t in call()} & {t.data_ptr() for t in mine}, name
+        stream[0] = 7
+    for first, (call, _) in _table_calls(dev).items():
+        A._TABLES = A._TableCache()
+        kept = call()
+        for T in range(1, 400):  # more shapes than are kept; this one is used all along
+            stream[0] = 7 + T % 3
+            A._token_tables(5, T + 10, dev)
+            stream[0] = 7
+            assert all(a is b for a, b in zip(call(), kept, strict=True)), (first, T)
+        held = A._TABLES.held
+        assert len(held) == A._TABLES.max_tables
+        assert A._TABLES.bytes == sum(t.nbytes for ts, _ in held.values() for t in ts)
+    A._TABLES = A._TableCache(max_bytes=5000)
+    for T in (100, 300, 10, 20, 2000, 30):
+        assert A._token_tables(1, T, dev)[1].numel() == T
+        assert A._TABLES.bytes <= 5000 or len(A._TABLES.held) == 1
+    assert [k[-1] for k in A._TABLES.held] == [30]
+
+
+def test_tables_of_two_threads_on_one_stream(monkeypatch):
+    """Two threads that miss together each get whole tables; one pair is kept
+    and its bytes are counted once."""
+    import threading
+
+    monkeypatch.setattr(A, "_raw_stream", lambda device: 7)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(A, "_TABLES", A._TableCache())
+    gate, got = threading.Barrier(2), []
+
+    def build():
+        gate.wait(timeout=30)
+        return (torch.arange(4),)
+
+    def call():
+        got.append(A._cached(torch.device("cpu"), ("x", 1), build))
+
+    ts = [threading.Thread(target=call) for _ in range(2)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join(timeout=30)
+    assert len(got) == 2 and all(torch.equal(g[0], torch.arange(4)) for g in got)
+    assert len(A._TABLES.held) == 1 and A._TABLES.bytes == 32

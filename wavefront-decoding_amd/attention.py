@@ -37,6 +37,8 @@ other than float32 / bfloat16, head sizes other than 64 / 128).
 from __future__ import annotations
 
 import math
+import threading
+from collections import OrderedDict
 
 import torch
 
@@ -68,25 +70,60 @@ def backend() -> str:
     return _BACKEND
 
 
-_TABLES: dict[tuple, tuple[torch.Tensor, ...]] = {}
+class _TableCache:
+    """Index tables by (device, stream, form, shape), the least recently used
+    dropped past `max_tables` entries or `max_bytes`. A table is built, read
+    and freed on one stream, so whatever the caching allocator makes of a
+    dropped one's memory is ordered behind its last reader."""
+
+    def __init__(self, max_tables: int = 256, max_bytes: int = 16 << 20):
+        self.max_tables, self.max_bytes = max_tables, max_bytes
+        self.lock = threading.Lock()
+        self.held: OrderedDict[tuple, tuple[tuple[torch.Tensor, ...], int]] = OrderedDict()
+        self.bytes = 0
+
+    def get(self, key: tuple) -> tuple[torch.Tensor, ...] | None:
+        with self.lock:
+            t = self.held.get(key)
+            if t is None:
+                return None
+            self.held.move_to_end(key)
+            return t[0]
+
+    def put(self, key: tuple, tables: tuple[torch.Tensor, ...]) -> None:
+        dropped = []  # freed after the lock
+        size = sum(t.nbytes for t in tables)
+        with self.lock:
+            if key in self.held:  # another thread on the same stream was first
+                dropped.append(self.held.pop(key))
+                self.bytes -= dropped[-1][1]
+            self.held[key] = (tables, size)
+            self.bytes += size
+            while len(self.held) > 1 and (len(self.held) > self.max_tables or self.bytes > self.max_bytes):
+                dropped.append(self.held.popitem(last=False)[1])
+                self.bytes -= dropped[-1][1]
 
 
-def _cached(key, build):
-    """The tables `build` makes on the device, kept by `key`. A stream under
-    capture gets tables of its own: built inside the capture, so that the
-    graph owns their memory and replays never read a table dropped since."""
-    if torch.cuda.is_current_stream_capturing():
-        return build()
-    t = _TABLES.get(key)
-    if t is None:
-        if len(_TABLES) > 256:
-            _TABLES.clear()
-        t = _TABLES[key] = build()
-    return t
+_TABLES = _TableCache()
 
 
 def _raw_stream(device: torch.device) -> int:
     return torch._C._cuda_getCurrentRawStream(device.index)
+
+
+def _cached(device: torch.device, key: tuple, build):
+    """The tables `build` makes on the device, kept for the current stream's
+    next calls with this key. A stream under capture gets tables of its own:
+    built inside the capture, so that the graph owns their memory and replays
+    never read a table dropped since."""
+    if torch.cuda.is_current_stream_capturing():
+        return build()
+    key = (device, _raw_stream(device), *key)
+    t = _TABLES.get(key)
+    if t is None:
+        t = build()
+        _TABLES.put(key, t)
+    return t
 
 
 def _scale(Dh: int) -> float:
@@ -101,7 +138,7 @@ def _dense_rows(B: int, Tq: int, Tk: int, causal: bool, device) -> tuple[torch.T
         kv = torch.arange(Tk - Tq + 1, Tk + 1, dtype=torch.int32, device=device).clamp_(min=0)
         return base, kv.expand(B, Tq).reshape(-1)
 
-    return _cached(("dense", B, Tq, Tk, causal, str(device)), build)
+    return _cached(device, ("dense", B, Tq, Tk, causal), build)
 
 
 def _prefill_segments(B: int, Tq: int, Tk: int, device):
@@ -110,7 +147,7 @@ def _prefill_segments(B: int, Tq: int, Tk: int, device):
                 torch.arange(B + 1, dtype=torch.int32, device=device).mul_(Tq),
                 torch.full((B,), Tk - Tq, dtype=torch.int32, device=device))
 
-    return _cached(("prefill", B, Tq, Tk, str(device)), build)
+    return _cached(device, ("prefill", B, Tq, Tk), build)
 
 
 def _shared_rows(total_q: int, nseg: int, max_k: int, H: int, Hkv: int, Dh: int) -> bool:
@@ -135,7 +172,7 @@ def _dense_offsets(B: int, Tq: int, Tk: int, device):
         s = torch.arange(B + 1, dtype=torch.int32, device=device)
         return s * Tq, s * Tk
 
-    return _cached(("dense_cu", B, Tq, Tk, device, _raw_stream(device)), build)
+    return _cached(device, ("offsets", B, Tq, Tk), build)
 
 
 def attn_dense(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, causal: bool) -> torch.Tensor:
@@ -209,8 +246,7 @@ def attn_varlen_q1_padded(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu_
     [cu_k[i], cu_k[i+1]) -- the result of the reference's padded form."""
     n = q.shape[0]
     ops._need_cuda(q)
-    cu_q = _cached(("q1", n, str(q.device)),
-                   lambda: (torch.arange(n + 1, dtype=torch.int32, device=q.device),))[0]
+    cu_q = _cached(q.device, ("q1", n), lambda: (torch.arange(n + 1, dtype=torch.int32, device=q.device),))[0]
     return attn_varlen(q, k, v, cu_q, cu_k, 1, max_k, causal=False)
 
 
@@ -238,11 +274,9 @@ def _fused_qkv_weight(attn):
 
 def _token_tables(B: int, T: int, device):
     """(positions 0..T-1 of every batch row, int32; row numbers, int64) of B * T
-    packed tokens. One pair per shape and stream (a pair that the table drops is
-    reused in the order of the stream that reads it)."""
-    return _cached(("tokens", B, T, device, _raw_stream(device)),
-                   lambda: (torch.arange(T, dtype=torch.int32, device=device).repeat(B),
-                            torch.arange(B * T, dtype=torch.int64, device=device)))
+    packed tokens."""
+    return _cached(device, ("tokens", B, T), lambda: (torch.arange(T, dtype=torch.int32, device=device).repeat(B),
+                                                      torch.arange(B * T, dtype=torch.int64, device=device)))
 
 
 def _rope_tables(freqs, B: int, T: int, Dh: int, device):
