@@ -7,6 +7,7 @@ import torch
 
 from wavefront_decoding_amd import _lib
 from wavefront_decoding_amd import attention as A
+from wavefront_decoding_amd import ops
 
 
 def test_backend_names():
@@ -136,3 +137,27 @@ def test_tables_of_two_threads_on_one_stream(monkeypatch):
         t.join(timeout=30)
     assert len(got) == 2 and all(torch.equal(g[0], torch.arange(4)) for g in got)
     assert len(A._TABLES.held) == 1 and A._TABLES.bytes == 32
+
+
+def test_split_workspace_belongs_to_its_stream(monkeypatch):
+    """The workspace attn_decode takes when none is passed: one per stream,
+    replaced only when a launch needs more; a capturing stream's is its own."""
+    stream, capturing = [7], [False]
+    monkeypatch.setattr(ops, "_raw_stream", lambda device: stream[0])
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing[0])
+    monkeypatch.setattr(ops, "_WS", type(ops._WS)())
+    ws = lambda n: ops.attn_workspace(n, 16, 128, 4096, "cpu")  # noqa: E731
+    a = ws(8)
+    assert a.numel() >= ops.attn_workspace_bytes(8, 16, 128, 4096) and ws(4) is a
+    stream[0] = 8
+    b = ws(8)
+    assert b is not a and ws(8) is b
+    capturing[0] = True
+    own = ws(8)
+    assert own is not b and own.numel() >= ops.attn_workspace_bytes(8, 16, 128, 4096) and ws(8) is not own
+    capturing[0] = False
+    assert ws(16).numel() >= ops.attn_workspace_bytes(16, 16, 128, 4096)
+    for s in range(100):
+        stream[0] = s
+        ws(1)
+    assert len(ops._WS) == ops._MAX_WORKSPACES

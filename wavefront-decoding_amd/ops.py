@@ -16,6 +16,7 @@ from __future__ import annotations
 
 import ctypes
 import math
+from collections import OrderedDict
 
 import torch
 
@@ -119,22 +120,33 @@ def _prep_args(n: int, D: int, dtype, *, r_in=None, s_in=None, w_in=None, r_out=
 # ---------------------------------------------------------------------------
 # attention
 # ---------------------------------------------------------------------------
-_WS: dict[int, torch.Tensor] = {}
+_WS: OrderedDict[tuple, torch.Tensor] = OrderedDict()  # (device, stream) -> workspace
+_MAX_WORKSPACES = 32
 
 
 def attn_workspace_bytes(n: int, H: int, Dh: int, kv_len_max: int) -> int:
     return int(_lib.load().wfd_attn_workspace_bytes(n, H, Dh, kv_len_max))
 
 
+def _raw_stream(device: torch.device) -> int:
+    return torch._C._cuda_getCurrentRawStream(device.index if device.index is not None
+                                              else torch.cuda.current_device())
+
+
 def attn_workspace(n: int, H: int, Dh: int, kv_len_max: int, device) -> torch.Tensor:
-    """A reusable uint8 workspace large enough for this launch shape."""
+    """A uint8 workspace large enough for this launch shape: the current
+    stream's, kept and grown, so that launches in flight on two streams never
+    share one. A stream under capture gets a fresh one, which the graph owns."""
     need = attn_workspace_bytes(n, H, Dh, kv_len_max)
     dev = torch.device(device)
-    key = dev.index if dev.index is not None else torch.cuda.current_device()
+    if torch.cuda.is_current_stream_capturing():
+        return torch.empty(max(need, 16), dtype=torch.uint8, device=dev)
+    key = (dev, _raw_stream(dev))
     ws = _WS.get(key)
     if ws is None or ws.numel() < need:
-        ws = torch.zeros(max(need, 1 << 20), dtype=torch.uint8, device=dev)
-        _WS[key] = ws
+        ws = _WS[key] = torch.empty(max(need, 1 << 20), dtype=torch.uint8, device=dev)
+        if len(_WS) > _MAX_WORKSPACES:
+            _WS.popitem(last=False)
     return ws
 
 
