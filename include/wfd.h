@@ -175,11 +175,14 @@ int wfd_attn_varlen_rows(const int32_t* cu_q, const int32_t* cu_k, int nseg, int
  * (total_q, H, Dh)) attends keys of [cu_k[s], cu_k[s+1]) of the token-major k /
  * v (total_k, Hkv, Dh) -- the whole segment, or bottom-right causal, exactly
  * the keys wfd_attn_varlen_rows gives the row; a row without keys, or outside
- * every segment, is zero. The call for segments of several rows: up to 32 /
+ * every segment, is zero. The call for segments of several rows: up to 16 /
  * (H / Hkv) rows of a segment read each key together on MFMA, where
- * wfd_attn_decode reads a row's keys for that row alone. fp32 softmax and
- * sums; the probabilities enter the second product as two bf16 terms (16
- * significant bits). A row's bits depend on its own keys only. max_k >= every
+ * wfd_attn_decode reads a row's keys for that row alone. Its arithmetic is
+ * wfd_attn_decode's value for value (fp32 probabilities, sums and division), so
+ * a row has the bits that call gives it, whichever rows and segments ride along;
+ * where V holds infinities or NaN, a row gets those of the keys it attends and
+ * no others (wfd_attn_decode also multiplies the last attended key's V by zero
+ * to fill its tile, which turns an infinity there into NaN). max_k >= every
  * segment's key count sizes the grid. workspace >=
  * wfd_attn_varlen_workspace_bytes(...), 16-byte aligned; q, k, v and out too.
  * Replaces: fa4_attention.attn_varlen / _attn_varlen_torch

@@ -151,6 +151,76 @@ def test_attn_varlen_shared_rows_special_values(gpu):
     assert d <= 2.0 ** -8
 
 
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("H,Hkv,Dh", [(16, 16, 128), (16, 8, 128), (16, 4, 128), (4, 4, 64), (4, 2, 64), (8, 2, 64)])
+def test_attn_varlen_rows_keep_their_bits(gpu, causal, H, Hkv, Dh):
+    """A row of a packed call has the bits of that row decoded alone, whatever
+    else the call holds: short calls, calls of many rows, other segments around
+    it, at the edges of row tiles (16 / G rows), key tiles and splits, with
+    scores from flat to so steep that probabilities underflow."""
+    T = 16 // (H // Hkv)
+    probe = [(T, 31), (T + 1, 33), (1, 64), (2, 1), (2 * T - 1, 1024), (3, 1025), (T, 2100), (5, 2), (3, 65)]
+    many = probe + [(40, 50 + i) for i in range(1400 // (40 * Hkv) + 12)]
+    nq, nk = (sum(x[i] for x in many) for i in (0, 1))
+    g = torch.Generator().manual_seed(H + Hkv + Dh + causal)
+    mk = lambda r, h: torch.randn(r, h, Dh, generator=g).to(torch.bfloat16).to(gpu)  # noqa: E731
+    q, k, v = mk(nq, H), mk(nk, Hkv), mk(nk, Hkv)
+    q *= torch.logspace(-2, 1.3, nq, device=gpu)[torch.randperm(nq, generator=g).to(gpu), None, None].to(q.dtype)
+    off = lambda x: torch.tensor(np.concatenate([[0], np.cumsum(x)]), dtype=torch.int32, device=gpu)  # noqa: E731
+    print(f"[attn_varlen bits] causal={causal} H={H} Hkv={Hkv} Dh={Dh}", flush=True)
+
+    def call(segs, q_, k_, v_, fn):
+        cq, ck, mk_ = off([a for a, _ in segs]), off([b for _, b in segs]), max(b for _, b in segs)
+        return fn(q_, k_, v_, cq, ck, max(a for a, _ in segs), mk_)
+
+    def rows(q_, k_, v_, cq, ck, mq, mk_):
+        rb, kl = ops.attn_varlen_rows(cq, ck, q_.shape[0], causal=causal)
+        return ops.attn_decode(q_, k_, v_, rb, kl, kv_len_max=mk_)
+
+    api = lambda *a: A.attn_varlen(*a, causal=causal)  # noqa: E731
+    shared = lambda q_, k_, v_, cq, ck, mq, mk_: ops.attn_varlen(q_, k_, v_, cq, ck, max_k=mk_, causal=causal)  # noqa: E731
+    assert A._shared_rows(nq, len(many), 2100, H, Hkv, Dh)
+    want = call(many, q, k, v, rows)
+    assert torch.equal(call(many, q, k, v, shared), want)
+    assert torch.equal(call(many, q, k, v, api), want)
+    q0 = k0 = 0
+    for a, b in probe:
+        args = q[q0: q0 + a], k[k0: k0 + b], v[k0: k0 + b]
+        for fn in (api, shared):
+            assert torch.equal(call([(a, b)], *args, fn), want[q0: q0 + a]), (a, b)
+        last = call([(1, b)], args[0][-1:], *args[1:], api)  # bottom-right: the segment's last row by itself
+        assert torch.equal(last, want[q0 + a - 1: q0 + a]), (a, b)
+        q0, k0 = q0 + a, k0 + b
+    if not causal:  # a dense call of many rows: one segment per batch row
+        B, Tq, Tk = 3, 1600 // Hkv, 70
+        d = [x[: B * t].view(B, t, -1, Dh) for x, t in ((mk(B * Tq, H), Tq), (k, Tk), (v, Tk))]
+        assert A._shared_rows(B * Tq, B, Tk, H, Hkv, Dh)
+        out = A.attn_dense(*d, causal=False)
+        for i in (0, 7, Tq - 1):
+            assert torch.equal(A.attn_dense(d[0][:, i: i + 1], *d[1:], causal=False), out[:, i: i + 1])
+
+
+@pytest.mark.parametrize("Hkv,Dh", [(2, 128), (1, 128), (2, 64)])
+def test_attn_varlen_special_values_stay_with_their_rows(gpu, Hkv, Dh):
+    """Infinities and NaN in V change no bit of a row that does not attend them,
+    in the key tile that holds them too, nor another column of one that does."""
+    g = torch.Generator().manual_seed(4)
+    n, H = 90, 2
+    q, k, v = (torch.randn(n, h, Dh, generator=g).to(torch.bfloat16).to(gpu) for h in (H, Hkv, Hkv))
+    cu = torch.tensor([0, n], dtype=torch.int32, device=gpu)
+    plain = ops.attn_varlen(q, k, v, cu, cu, max_k=n, causal=True)
+    v[40, 0, 5] = float("inf")
+    v[70, Hkv - 1, 7] = float("nan")
+    v[71, Hkv - 1, 8] = float("-inf")
+    got = ops.attn_varlen(q, k, v, cu, cu, max_k=n, causal=True)
+    inf_heads, last_heads = slice(0, H // Hkv), slice(H - H // Hkv, H)
+    assert (got[40:, inf_heads, 5] == float("inf")).all()
+    assert torch.isnan(got[70:, last_heads, 7]).all() and (got[71:, last_heads, 8] == float("-inf")).all()
+    clean = torch.ones_like(got, dtype=torch.bool)
+    clean[40:, inf_heads, 5] = clean[70:, last_heads, 7] = clean[71:, last_heads, 8] = False
+    assert torch.equal(got[clean], plain[clean])
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_attn_varlen_q1_padded_matches_oracle(gpu, dtype):
     lens = [1, 64, 300, 1025, 7]

@@ -9,17 +9,16 @@ runs a HIP kernel of libwfd.so on torch's current stream:
 
   attn_dense      bf16 causal with Tq <= Tk (a prompt, bottom-right aligned):
                   the MFMA prefill kernel (wfd_attn_prefill), one segment per
-                  batch row; other bf16 calls of many rows: the varlen kernel
-                  (wfd_attn_varlen), one segment per batch row; otherwise the
-                  decode kernel (wfd_attn_decode) with one (row base, key
-                  count) entry per query row
+                  batch row; otherwise as attn_varlen, one segment per batch
+                  row
   attn_cutoff_multi  the decode kernel with key count = qpos + 1
-  attn_varlen     bf16 with at least two rows per segment and rows enough
-                  (_shared_rows): the varlen kernel, whose workgroups read a
-                  key once for up to 32 / (H / Hkv) rows of its segment;
-                  otherwise the decode kernel over the packed K / V (token-major), its row tables
-                  expanded from cu_q / cu_k on the device
-                  (wfd_attn_varlen_rows). Nothing is read back to the host
+  attn_varlen     the decode kernel (wfd_attn_decode) over the packed K / V
+                  (token-major), with one (row base, key count) entry per query
+                  row, expanded from cu_q / cu_k on the device
+                  (wfd_attn_varlen_rows); bf16 calls with rows enough
+                  (_shared_rows): wfd_attn_varlen, whose workgroups read a key
+                  once for up to 16 / (H / Hkv) rows of its segment, with the
+                  decode kernel's bits. Nothing is read back to the host
   attn_varlen_q1_padded  attn_varlen with one query row per segment (the
                   reference pads each to two causal rows to steer FA2's tile
                   choice; the decode kernel has no such template switch, and
@@ -151,20 +150,22 @@ def _prefill_segments(B: int, Tq: int, Tk: int, device):
 
 
 def _shared_rows(total_q: int, nseg: int, max_k: int, H: int, Hkv: int, Dh: int) -> bool:
-    """Whether the kernel that reads a key once for all rows of a segment
+    """Whether the kernel that reads a key once for several rows of a segment
     (wfd_attn_varlen) takes this bf16 call: Dh 64 / 128, 1, 2 or 4 query heads
-    per kv head, and rows enough to gain by it. The decode kernel's workgroups
-    (one per row, kv head and 1024 keys) repeat the segment's reads but spread
-    over more CUs: it wins below two rows a segment and while its launch is at
-    most one round of resident workgroups, two per CU, or one with Dh 64 or (a
-    little earlier) with four query heads, by LDS. us, decode against this
-    kernel: 16 heads, 4 segments of 8 / 16 rows x 1000 keys (512 / 1024 workgroups)
-    19 / 32 against 19 / 19, 48 segments of 2 rows 87 against 73; 16 heads over 4
-    kv heads, 16 segments of 2 / 4 / 8 rows x 1000 keys 22 / 22 / 39 against 19; 4 over
-    2 heads of 64, 16 segments of 8 / 16 rows (256 / 512) 12.5 / 16.2 against 13.7."""
+    per kv head, and rows enough to gain by it. Both kernels give a row the
+    same bits, so the line is a matter of time alone. The decode kernel's
+    workgroups (one per row, kv head and 1024 keys) repeat the segment's reads
+    but are short, and few rows leave most of the other's 16-row products
+    empty: it wins below two rows a segment and up to some rounds of its
+    workgroups: three of 256 at Dh 128, one with four query heads per kv head
+    (which it takes longest over), four of the half as long ones at Dh 64. us,
+    decode against this kernel, by workgroups: Dh 128, 16 heads: 384 16.1 / 24.2, 736
+    13.0 / 13.3, 1568 21 / 14 and 43 / 27, 4960 99 / 52, 32384 735 / 168; 16 heads
+    over 4: 164 10.1 / 13.4, 268 24.6 / 23.0, 392 33 / 26, 8096 460 / 122; Dh 64, 4
+    heads: 512 9.7 / 14.1, 704 24 / 31, 1480 15.6 / 11.2, 8096 111 / 45."""
     if total_q < 2 * nseg or Dh not in (64, 128) or Hkv <= 0 or H not in (Hkv, 2 * Hkv, 4 * Hkv):
         return False
-    return total_q * Hkv * ((max_k + 1023) // 1024) > (256 if Dh == 64 else 191 if H == 4 * Hkv else 512)
+    return total_q * Hkv * ((max_k + 1023) // 1024) > (1024 if Dh == 64 else 256 if H == 4 * Hkv else 768)
 
 
 def _dense_offsets(B: int, Tq: int, Tk: int, device):

@@ -1,53 +1,64 @@
-// Packed varlen attention for segments of several query rows (bf16), on MFMA.
+// Packed varlen attention for segments of several query rows (bf16), on MFMA,
+// with the decode kernel's bits.
 //
 // Replaces: fa4_attention.attn_varlen / _attn_varlen_torch
 //   (src/decoding/fa4_attention.py:301-317,348-366) where a segment brings more
 //   than one row: chunked prompts, a coda's verifies, re-entered tokens.
 //
 // Same operation as the row form (varlen row tables + wfd_attn_decode): query
-// row r of a segment attends the segment's first kv_len[r] keys; softmax and
-// sums in fp32. The row form streams a row's whole prefix once per row; here a
-// workgroup owns a tile of 32 / G rows of one segment (G = H / Hkv query heads
-// per kv head: 32 (row, head) pairs, one per lane column of a 32x32 MFMA) and
-// one kv head, and reads each key once for all of them.
+// row r of a segment attends the segment's first kv_len[r] keys. The row form
+// streams a row's whole prefix once per row; here a workgroup owns a tile of
+// 16 / G rows of one segment (G = H / Hkv query heads per kv head: 16 (row, head)
+// pairs, one per lane column) and one kv head, and reads each key once for all.
 //
-// What bounds it: with up to 32 rows per key the call is a stream of K and V
-// (at 48 segments of 1-64 rows over 100-2048 keys x 16 heads x 128: 394 MB),
-// so the layout keeps loads in flight: 4 waves take the 32-key tiles of a
-// 1024-key split round-robin, each with its own LDS block and no barrier in the
-// loop; a tile's 16 KB are loaded into registers (whole key rows, 1 KB per
-// instruction) while the tile before it is computed. Two workgroups per CU fit
-// by LDS (80 KB each at Dh 128, Q's fragments among them: in registers they made
-// the loop spill), so one streams while the other merges. That shape takes 124
-// us (the tables 5, this kernel 111, the merge of splits 10; 3.5 TB/s) against
-// 720 us for the row form; what is left is the ragged last round of 1540
-// workgroups over 512 places. Two S^T chains instead of one changed nothing.
+// Arithmetic: exactly attn_split_kernel's, value for value, so a row has the
+// same bits whichever kernel a call takes and whichever rows ride along:
+//  * scores on the same 16x16x32 bf16 product in the same k order, formed
+//    transposed (K as the A operand), which leaves a lane with scores of one
+//    (row, head) pair: its softmax state is one register each;
+//  * the same tile per wave (tile t of a 1024-key split belongs to wave t % 8),
+//    and a tile's sum of probabilities in the row form's order: over 16-key
+//    blocks, then the xor 8, 4, 2, 1 butterfly over the key within the block;
+//  * P.V in fp32 on v_mfma_f32_16x16x4_f32, which is the chain
+//    fma(a3,b3,fma(a2,b2,fma(a1,b1,fma(a0,b0,c)))) bit for bit, denormals,
+//    infinities and NaN included (checked on the device against fmaf over 7
+//    distributions x 10^6 sums: no difference, every other order differs). The
+//    row form's lane vg adds keys RG k + vg, k = 0, 1, ..; here that chain is
+//    an accumulator of its own, four keys per product (lane group = k), and the
+//    keys of a tile are permuted so that a lane's probabilities are the
+//    product's B operand in place;
+//  * the chains' and the waves' merge in the same order, splits in split order
+//    (attn_combine_kernel).
 //
-// Arithmetic: S^T = K Q^T and O^T = V^T P^T on v_mfma_f32_32x32x16_bf16, V^T
-// read from the row-major tile with the transposing LDS read, keys permuted
-// inside a tile so that the S^T accumulators are the P^T operand in place
-// (lane half hf, register rr: key 16 (rr / 8) + 8 hf + rr % 8). The
-// probabilities enter the second product as two bf16 terms, p = hi + lo (16
-// significant bits), each its own MFMA into the same fp32 sum, so they are not
-// rounded to bf16: the output's error against float64 is that of the row form
-// (1.7e-3, the bf16 output rounding; with hi alone 2.0e-3). A row's bits depend
-// on its own keys only, not on its tile, its column or the other segments: key
-// tiles go to waves and splits by key index, masked keys add exact zeros.
-// Waves merge through LDS in wave order, splits in split order
-// (attn_combine_kernel).
+// What bounds it: issue. A tile of 16 pairs x 32 keys x 128 columns is 64 fp32
+// products of 32 cycles, a third of the time of 48 segments of 1-64 rows over
+// 100-2048 keys x 16 heads x 128 (394 MB of K and V): 168 us (the tables 5, this
+// kernel 152, the merge of splits 10) against 720 for the row form. The chains
+// take 128 registers, so a CU holds 8 waves: as two workgroups of 4 waves with
+// two parts each, so that one's loads and merge run under the other's products
+// (one workgroup of 8 waves: 209 us; with the merge's factors computed once per
+// output, 182). K and V of the next tile are loaded as soon as the registers of
+// this one's are free.
 #include "attn_combine.h"
 
 namespace wfd {
 
-constexpr int kRowsCols = 32;   // (row, head) pairs per workgroup
-constexpr int kRowsWaves = 4;
-constexpr int kRowsKeys = 32;   // keys per tile
+constexpr int kRowsCols = 16;   // (row, head) pairs per workgroup
+constexpr int kRowsParts = 8;   // attn_split_kernel's waves: part w sums tiles w, w + 8, ..
+constexpr int kRowsWaves = 4;   // each takes parts w and w + 4 in turn
 
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-__device__ __forceinline__ f32x16 rows_mfma(const u32x4& a, const u32x4& b, f32x16 acc) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), acc,
-                                                 0, 0, 0);
+// (x of the lane with bit 5 / bit 4 of its number clear, x of the one with it set), the
+// other bits the lane's own: a butterfly step's two terms without the LDS
+struct Pair {
+  float a, b;
+};
+__device__ __forceinline__ Pair pair32(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return {__uint_as_float(r[0]), __uint_as_float(r[1])};
+}
+__device__ __forceinline__ Pair pair16(float x) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return {__uint_as_float(r[0]), __uint_as_float(r[1])};
 }
 
 // Tiles of at most `qt` rows, none across a segment boundary: tile i holds rows
@@ -111,22 +122,21 @@ __global__ __launch_bounds__(64 * kRowsWaves) __attribute__((amdgpu_waves_per_eu
     const int64_t* __restrict__ row_base, const int32_t* __restrict__ kv_len, const int32_t* __restrict__ tile_first,
     float* __restrict__ part_o, float* __restrict__ part_ml, bf16_t* __restrict__ out, int H, int Hkv, int max_splits,
     float scale_log2) {
-  constexpr int V = 8;
   constexpr int NW = kRowsWaves;
-  constexpr int QT = kRowsCols / G;        // rows per tile
-  constexpr int NDS = DH / 16;             // MFMA k-steps over Dh
-  constexpr int NDB = DH / 32;             // 32-row blocks of O^T
-  constexpr int VRP = DH + 32;             // padded LDS row of V (elements): spreads a transposing read over all banks
-  constexpr int CPR = DH / V;              // 16-byte pieces of a key row
-  constexpr int NCH = kRowsKeys * CPR / 64;  // K (and V) pieces per lane per tile
-  constexpr int PW = NDB * 16 + 2;         // floats a lane parks for the merge
-  constexpr int kWaveLds = kRowsKeys * (DH + VRP) * (int)sizeof(bf16_t);
-  static_assert(NW * kWaveLds >= NW * PW * 64 * (int)sizeof(float), "park area");
-  static_assert(NDS % NW == 0, "Q fragments staged by wave");
-  static_assert(NDB <= NW && kRowsCols % G == 0, "merge split");
-  static_assert(kRowsKeys * DH * sizeof(bf16_t) >= kRowsKeys * 32 * sizeof(float), "P in the K tile's LDS");
-  __shared__ __align__(16) unsigned char lds[NW * kWaveLds];
-  __shared__ __align__(16) u32x4 q_lds[NDS][64];  // Q fragments: 32 registers a lane fewer, or the loop spills
+  constexpr int NP = kRowsParts;
+  constexpr int QT = kRowsCols / G;   // rows per tile
+  constexpr int TK = DH == 64 ? 64 : 32;  // keys per tile, as attn_split_kernel
+  constexpr int RG = 512 / DH;        // P.V chains (attn_split_kernel's V row groups)
+  constexpr int NJ = TK / 16;         // 16-key blocks of S^T
+  constexpr int NDS = DH / 32;        // MFMA k-steps over Dh
+  constexpr int NB = DH / 16;         // 16-column blocks of O^T: block b holds columns NB i + b
+  constexpr int NS = TK / (4 * RG);   // products per chain and tile
+  constexpr int PW = NB / 2;          // 32-bit words of a lane's V piece
+  constexpr int OP = DH + 4;          // padded row of the merge area
+  static_assert(NJ * 4 == NS * RG && NS == 2, "score registers are the P.V operands");
+  __shared__ __align__(16) float o_lds[NP][kRowsCols][OP];
+  __shared__ float m_lds[NP][kRowsCols];
+  __shared__ float l_lds[NP][kRowsCols];
 
   const int g = blockIdx.x % Hkv;
   const int tile = blockIdx.x / Hkv;
@@ -136,15 +146,13 @@ __global__ __launch_bounds__(64 * kRowsWaves) __attribute__((amdgpu_waves_per_eu
   if (nr <= 0) return;  // empty tile (uniform)
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const int col = lane & 31;  // this lane's (row, head) pair
-  const int hf = lane >> 5;
+  const int col = lane & 15;  // this lane's (row, head) pair; as an A row: its key or column group
+  const int grp = lane >> 4;
   const bool real = col / G < nr;
-  const int row = r0 + (real ? col / G : 0);
-  const int head = g * G + col % G;
-  const int lim = real ? max(kv_len[row], 0) : 0;  // keys [0, lim)
+  const int lim = real ? max(kv_len[r0 + col / G], 0) : 0;  // keys [0, lim)
   int maxlen = lim, minlen = real ? lim : 0x7fffffff;
 #pragma unroll
-  for (int m = 16; m >= 1; m >>= 1) {
+  for (int m = 8; m >= 1; m >>= 1) {
     maxlen = max(maxlen, __shfl_xor(maxlen, m, 64));
     minlen = min(minlen, __shfl_xor(minlen, m, 64));
   }
@@ -153,7 +161,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) __attribute__((amdgpu_waves_per_eu
   const int kbeg = split * kAttnSplit;
   if (split > 0 && kbeg >= maxlen) return;  // uniform over the workgroup
   const int nkeys = max(min(maxlen, kbeg + kAttnSplit) - kbeg, 0);  // of this split
-  const int nt = (nkeys + kRowsKeys - 1) / kRowsKeys;
+  const int nt = (nkeys + TK - 1) / TK;
 
   // K / V of this kv head from key kbeg; the resources end at the split's last
   // key, so loads of later keys read zeros and send nothing to memory
@@ -164,223 +172,243 @@ __global__ __launch_bounds__(64 * kRowsWaves) __attribute__((amdgpu_waves_per_eu
                                                                       0x00020000);
   const __amdgpu_buffer_rsrc_t vr = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(vc + hb), (short)0, span,
                                                                       0x00020000);
-  bf16_t* const kl = reinterpret_cast<bf16_t*>(lds + wave * kWaveLds);
-  bf16_t* const vl = kl + kRowsKeys * DH;
-  // K rows unpadded, 16-byte pieces XORed by the row: 16 rows' reads of one piece
-  // (and a row's 16 stores) touch every bank once
-  auto k_at = [](int key, int piece) {
-    return (key * CPR + (piece ^ (CPR == 16 ? key & 15 : (key >> 1) & (CPR - 1)))) * V;
+
+  // Score block j, MFMA row i = 4 grp + r is key RG (4 s + grp) + vg of the tile
+  // for the product (s, vg) = (4 j + r) / RG, (4 j + r) % RG: the row form's
+  // chain vg at its step k = 4 s + grp
+  auto key_of = [](int j, int i) {
+    return RG * (4 * (4 * j / RG) + (i >> 2)) + (4 * j) % RG + (i & 3);
   };
 
-  // Q as the MFMA B operand: column col, dims 16 k + 8 hf + (0..7)
+  u32x4 kreg[NJ][NDS];
+  uint32_t vreg[NS * RG][PW];
+  const uint32_t k_lane = (uint32_t)key_of(0, col) * rsb + (uint32_t)grp * 16u;
+  const uint32_t v_lane = (uint32_t)(RG * grp) * rsb + (uint32_t)(col * NB * 2);
+  auto fetch_k = [&](int t) {
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const uint32_t off = k_lane + (uint32_t)(t * TK + key_of(j, 0)) * rsb;
+#pragma unroll
+      for (int s = 0; s < NDS; ++s) kreg[j][s] = buf_ld16(kr, off + s * 64);
+    }
+  };
+  auto fetch_v = [&](int t, int x) {  // piece x = (s, vg): NB columns of key RG (4 s + grp) + vg
+    const uint32_t off = v_lane + (uint32_t)(t * TK + 4 * RG * (x / RG) + x % RG) * rsb;
+    if constexpr (PW == 4) {
+      const u32x4 w = buf_ld16(vr, off);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) vreg[x][e] = w[e];
+    } else {
+      typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+      const u32x2 w = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(vr, off, 0, 0));
+      vreg[x][0] = w[0];
+      vreg[x][1] = w[1];
+    }
+  };
+
+  auto lo_special = [](uint32_t w) { return (w & 0x7f80u) == 0x7f80u; };  // infinite or NaN
+  auto hi_special = [](uint32_t w) { return (w & 0x7f800000u) == 0x7f800000u; };
+
+  fetch_k(wave);
+  // Q as the B operand: column col, dims 32 s + 8 grp + (0..7)
+  u32x4 qf[NDS];
   {
-    const bf16_t* qp = q + ((int64_t)row * H + head) * DH + hf * V;
+    const bf16_t* qp = q + ((int64_t)(r0 + (real ? col / G : 0)) * H + g * G + col % G) * DH + grp * 8;
 #pragma unroll
-    for (int i = 0; i < NDS / NW; ++i) {
-      const int k = wave * (NDS / NW) + i;
-      q_lds[k][lane] = ld16(qp + k * 16);
-    }
+    for (int s = 0; s < NDS; ++s) qf[s] = real ? ld16(qp + s * 32) : zero16();
   }
-  // key (within a tile) of MFMA row col: the permutation above
-  const int krow = 16 * ((col >> 3) >> 1) + 8 * ((col >> 2) & 1) + 4 * ((col >> 3) & 1) + (col & 3);
+#pragma unroll
+  for (int x = 0; x < NS * RG; ++x) fetch_v(wave, x);
+#pragma unroll 1
+  for (int part = wave; part < NP; part += NW) {
+    float mrun = -INFINITY, lrun = 0.f;
+    f32x4 o[RG][NB];  // O^T by chain: columns NB (4 grp + r) + b of pair col
+#pragma unroll
+    for (int c = 0; c < RG; ++c)
+#pragma unroll
+      for (int b = 0; b < NB; ++b) o[c][b] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  u32x4 kreg[NCH], vreg[NCH];
-  const uint32_t lane_off = (uint32_t)(lane / CPR) * rsb + (uint32_t)(lane % CPR) * 16u;
-  auto fetch = [&](int t) {
+    for (int t = part; t < nt; t += NP) {  // uniform over the wave; no barrier in the loop
+      const int tn = t + NP < nt || part >= NW ? t + NP : part + NW;  // the next tile: of this part, or the wave's other one
+      const int t0 = kbeg + t * TK;
+      f32x4 p[NJ];
 #pragma unroll
-    for (int i = 0; i < NCH; ++i) {
-      const uint32_t off = lane_off + (uint32_t)(t * kRowsKeys + i * (64 / CPR)) * rsb;
-      kreg[i] = buf_ld16(kr, off);
-      vreg[i] = buf_ld16(vr, off);
-    }
-  };
-  // V^T fragment of d-block db, key step k (see the prefill kernel): two
-  // transposing reads of 4 keys x 16 columns per 16-lane group
-  const int tg = lane >> 4, ti = lane & 15;
-  const int v_lane = ((tg >> 1) * 8 + (ti >> 2)) * VRP + 16 * (tg & 1) + 4 * (ti & 3);
-  auto vt_frag = [&](int db, int k) {
-    typedef short s16x4 __attribute__((ext_vector_type(4)));
-    typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-    typedef const __attribute__((address_space(3))) void* lds_ptr;
-    const bf16_t* p = vl + v_lane + 16 * k * VRP + 32 * db;
-    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(lds_ptr)p);
-    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(lds_ptr)(p + 4 * VRP));
-    const uint2 a = __builtin_bit_cast(uint2, lo), c = __builtin_bit_cast(uint2, hi);
-    return u32x4{a.x, a.y, c.x, c.y};
-  };
-
-  float mrun = -INFINITY, lrun = 0.f;
-  f32x16 o[NDB];
+      for (int j = 0; j < NJ; ++j) {
+        p[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int c = 0; c < NDB; ++c)
+        for (int s = 0; s < NDS; ++s) p[j] = mfma_step<bf16_t>(kreg[j][s], qf[s], p[j]);
+      }
+      fetch_k(tn);  // past the last tile: zeros, no traffic
+      {
+#pragma clang fp contract(off)
+        float mt = -INFINITY;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) o[c][r] = 0.f;
-
-  // Whether a V value of the lane's loaded tile is infinite or NaN. Such a tile
-  // leaves the matrix product (0 x infinity for a masked key or a zero low term
-  // would reach rows that the value does not belong to) and is added key by key.
-  auto v_special = [&]() {
-    typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
-    u16x2 m = {0, 0};
+        for (int j = 0; j < NJ; ++j)
 #pragma unroll
-    for (int i = 0; i < NCH; ++i)
+          for (int r = 0; r < 4; ++r) {
+            const float sv = t0 + key_of(j, 4 * grp) + r < lim ? p[j][r] * scale_log2 : -INFINITY;
+            p[j][r] = sv;
+            mt = fmaxf(mt, sv);
+          }
+        const Pair m32 = pair32(mt);
+        const Pair m16 = pair16(fmaxf(m32.a, m32.b));
+        mt = fmaxf(m16.a, m16.b);
+        const float mnew = fmaxf(mrun, mt);
+        const float corr = (mrun == -INFINITY) ? 0.f : exp2f(mrun - mnew);
+        mrun = mnew;
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        m = __builtin_elementwise_max(m, __builtin_bit_cast(u16x2, vreg[i][e] & 0x7f807f80u));
-    return m.x == 0x7f80 || m.y == 0x7f80;
-  };
-
-  fetch(wave);
-  __syncthreads();  // q_lds
-  for (int t = wave; t < nt; t += NW) {  // uniform over the wave; no barrier in the loop
-    // the LDS executes one wave's accesses in order: the previous tile's
-    // reads, these stores, this tile's reads
-    const bool special = __builtin_amdgcn_ballot_w64(v_special()) != 0;  // uniform
-    asm volatile("" ::: "memory");
+        for (int j = 0; j < NJ; ++j)
 #pragma unroll
-    for (int i = 0; i < NCH; ++i) {
-      const int c = lane + 64 * i;
-      *reinterpret_cast<u32x4*>(kl + k_at(c / CPR, c % CPR)) = kreg[i];
-      *reinterpret_cast<u32x4*>(vl + (c / CPR) * VRP + (c % CPR) * V) = vreg[i];
-    }
-    asm volatile("" ::: "memory");
-    fetch(t + NW);  // past the last tile: zeros, no traffic
-    f32x16 s;
+          for (int r = 0; r < 4; ++r) p[j][r] = (p[j][r] == -INFINITY) ? 0.f : exp2f(p[j][r] - mnew);
+        // the tile's sum, by key % 16 (c) over the tile's 16-key blocks, then the
+        // butterfly over c: xor 8, 4, 2, 1
+        float u[4];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) s[r] = 0.f;
+        for (int r = 0; r < 4; ++r) {
+          if constexpr (RG == 4) {  // c = 4 grp + r
+            const Pair v = pair32(p[0][r] + p[1][r]);
+            const Pair w = pair16(v.a + v.b);
+            u[r] = w.a + w.b;
+          } else {  // c = 8 (grp & 1) + 4 h + r, 16-key block 2 s + grp / 2
+            float w[2];
 #pragma unroll
-    for (int k = 0; k < NDS; ++k)
-      s = rows_mfma(*reinterpret_cast<const u32x4*>(kl + k_at(krow, 2 * k + hf)), q_lds[k][lane], s);
-    const int k0 = kbeg + t * kRowsKeys;
-    if (k0 + kRowsKeys > minlen) {  // some row's last key lies in or before this tile (uniform)
+            for (int h = 0; h < 2; ++h) {
+              const Pair s0 = pair32(p[h][r]), s1 = pair32(p[2 + h][r]);
+              const Pair v = pair16(((s0.a + s0.b) + s1.a) + s1.b);
+              w[h] = v.a + v.b;
+            }
+            u[r] = w[0] + w[1];
+          }
+        }
+        lrun = fmaf(lrun, corr, (u[0] + u[2]) + (u[1] + u[3]));
+        if (t != part && __builtin_amdgcn_ballot_w64(corr != 1.f)) {  // the first tile: o is 0
 #pragma unroll
-      for (int r = 0; r < 16; ++r)
-        if (k0 + 16 * (r >> 3) + 8 * hf + (r & 7) >= lim) s[r] = -INFINITY;
-    }
-    float mt = s[0];
+          for (int c = 0; c < RG; ++c)
 #pragma unroll
-    for (int r = 1; r < 16; ++r) mt = fmaxf(mt, s[r]);
-    mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
-    const float mnew = fmaxf(mrun, mt * scale_log2);
-    const float mref = mnew == -INFINITY ? 0.f : mnew;  // a row with no key so far: every p is 0
-    const float corr = __builtin_amdgcn_exp2f(mrun - mref);
-    float ls = 0.f;
+            for (int b = 0; b < NB; ++b)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      s[r] = __builtin_amdgcn_exp2f(fmaf(s[r], scale_log2, -mref));
-      ls += s[r];
-    }
-    ls += __shfl_xor(ls, 32, 64);
-    lrun = fmaf(lrun, corr, ls);
-    mrun = mnew;
-    if (__builtin_amdgcn_ballot_w64(corr != 1.f)) {
-#pragma unroll
-      for (int db = 0; db < NDB; ++db)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) o[db][r] *= corr;
-    }
-    if (special) {
-      // P through the K tile's LDS (its reads are done), one key at a time, then
-      // zeros in V's place for the products below
-      float* const pl32 = reinterpret_cast<float*>(kl);
-      asm volatile("" ::: "memory");
-#pragma unroll
-      for (int r = 0; r < 16; ++r) pl32[(16 * (r >> 3) + 8 * hf + (r & 7)) * 32 + col] = s[r];
-      asm volatile("" ::: "memory");
-      for (int key = 0; key < kRowsKeys && k0 + key < maxlen; ++key) {
-        const bool mine = k0 + key < lim;
-        const float p = mine ? pl32[key * 32 + col] : 0.f;
-#pragma unroll
-        for (int i = 0; i < 4 * NDB; ++i) {
-          const uint2 w = *reinterpret_cast<const uint2*>(vl + key * VRP + 8 * i + 4 * hf);
-          f32x16& oo = o[i >> 2];
-          const int b = 4 * (i & 3);
-          oo[b + 0] = fmaf(p, mine ? bf16_bits_to_f32(w.x & 0xffffu) : 0.f, oo[b + 0]);
-          oo[b + 1] = fmaf(p, mine ? bf16_bits_to_f32(w.x >> 16) : 0.f, oo[b + 1]);
-          oo[b + 2] = fmaf(p, mine ? bf16_bits_to_f32(w.y & 0xffffu) : 0.f, oo[b + 2]);
-          oo[b + 3] = fmaf(p, mine ? bf16_bits_to_f32(w.y >> 16) : 0.f, oo[b + 3]);
-          __builtin_amdgcn_sched_barrier(0);
+              for (int r = 0; r < 4; ++r) o[c][b][r] *= corr;
         }
       }
-      asm volatile("" ::: "memory");
+      // A tile in which some row's last key lies (uniform): 0 x infinity would
+      // reach rows that an infinite or NaN V value does not belong to. Such a value
+      // becomes 0 in the products and is added here to the pairs that attend it (to
+      // chain 0: which chain holds an infinity or a NaN changes nothing)
+      if (t0 + TK > minlen) {
 #pragma unroll
-      for (int i = 0; i < NCH; ++i) {
-        const int c = lane + 64 * i;
-        *reinterpret_cast<u32x4*>(vl + (c / CPR) * VRP + (c % CPR) * V) = zero16();
+        for (int x = 0; x < NS * RG; ++x) {
+          bool special = false;
+#pragma unroll
+          for (int e = 0; e < PW; ++e) special |= lo_special(vreg[x][e]) || hi_special(vreg[x][e]);
+          if (__builtin_amdgcn_ballot_w64(special) == 0) continue;
+#pragma unroll 1
+          for (int k = 0; k < 4; ++k) {  // key RG (4 s + k) + vg: held by lane group k
+            const float pk = __shfl(p[x / 4][x % 4], 16 * k + col, 64);
+            const bool mine = t0 + RG * (4 * (x / RG) + k) + x % RG < lim;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+              for (int e = 0; e < PW; ++e) {
+                const uint32_t w = __shfl(vreg[x][e], 16 * k + 4 * grp + r, 64);
+                if (mine && lo_special(w)) o[0][2 * e][r] = fmaf(pk, __uint_as_float(w << 16), o[0][2 * e][r]);
+                if (mine && hi_special(w)) o[0][2 * e + 1][r] = fmaf(pk, __uint_as_float(w & 0xffff0000u), o[0][2 * e + 1][r]);
+                __builtin_amdgcn_sched_barrier(0);
+              }
+          }
+#pragma unroll
+          for (int e = 0; e < PW; ++e) {
+            if (lo_special(vreg[x][e])) vreg[x][e] &= 0xffff0000u;
+            if (hi_special(vreg[x][e])) vreg[x][e] &= 0xffffu;
+          }
+        }
       }
-      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int x = 0; x < NS * RG; ++x) {
+#pragma unroll
+        for (int e = 0; e < PW; ++e) {
+          f32x4& lo = o[x % RG][2 * e];
+          f32x4& hi = o[x % RG][2 * e + 1];
+          lo = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(vreg[x][e] << 16), p[x / 4][x % 4], lo, 0, 0, 0);
+          hi = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(vreg[x][e] & 0xffff0000u), p[x / 4][x % 4], hi, 0, 0,
+                                                    0);
+        }
+        fetch_v(tn, x);
+      }
     }
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      // p = hi + lo, both bf16: P^T operand of key step k from registers 8k .. 8k + 7
-      u32x4 ph, pl;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float p0 = s[8 * k + 2 * e], p1 = s[8 * k + 2 * e + 1];
-        ph[e] = f32x2_to_bf16x2_bits(p0, p1);
-        pl[e] = f32x2_to_bf16x2_bits(p0 - __uint_as_float(ph[e] << 16), p1 - __uint_as_float(ph[e] & 0xffff0000u));
-      }
-#pragma unroll
-      for (int db = 0; db < NDB; ++db) {
-        const u32x4 vt = vt_frag(db, k);
-        o[db] = rows_mfma(vt, ph, o[db]);
-        o[db] = rows_mfma(vt, pl, o[db]);
-      }
-    }
-  }
 
-  // merge the waves in wave order: each parks its state (its own LDS block may
-  // be another wave's park area: barrier first), then wave db merges d-block db
-  __syncthreads();
-  float* const park = reinterpret_cast<float*>(lds);
-  {
-    float* p = park + wave * PW * 64 + lane;
+    // the chains in the row form's shuffle order, then the part leaves its state
 #pragma unroll
-    for (int db = 0; db < NDB; ++db)
+    for (int c = 1; c < RG; c <<= 1)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) p[(16 * db + r) * 64] = o[db][r];
-    p[16 * NDB * 64] = mrun;
-    p[(16 * NDB + 1) * 64] = lrun;
-  }
-  __syncthreads();
-  if (wave >= NDB) return;  // after the last barrier
-  const int db = wave;
-  float M = -INFINITY, L = 0.f, O[16];
+      for (int a = 0; a < RG; a += 2 * c)
 #pragma unroll
-  for (int w = 0; w < NW; ++w) M = fmaxf(M, park[(w * PW + 16 * NDB) * 64 + lane]);
+        for (int b = 0; b < NB; ++b) o[a][b] += o[a + c][b];
 #pragma unroll
-  for (int r = 0; r < 16; ++r) O[r] = 0.f;
+    for (int r = 0; r < 4; ++r)
 #pragma unroll
-  for (int w = 0; w < NW; ++w) {
-    const float* p = park + w * PW * 64 + lane;
-    const float mw = p[16 * NDB * 64];
-    const float f = mw == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mw - M);
-    L = fmaf(p[(16 * NDB + 1) * 64], f, L);
-#pragma unroll
-    for (int r = 0; r < 16; ++r) O[r] = fmaf(p[(16 * db + r) * 64], f, O[r]);
-  }
-  if (!real) return;
-  // register r: output column d = 32 db + 8 (r / 4) + 4 hf + r % 4
-  const int ns = min((lim + kAttnSplit - 1) / kAttnSplit, max_splits);
-  const int64_t oh = (int64_t)row * H + head;
-  if (ns <= 1) {
-    if (split > 0) return;
-    const float inv = L > 0.f ? 1.f / L : 0.f;  // a row without keys: zeros
-    bf16_t* op = out + oh * DH + 32 * db + 4 * hf;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      uint2 w;
-      w.x = f32x2_to_bf16x2_bits(O[4 * i] * inv, O[4 * i + 1] * inv);
-      w.y = f32x2_to_bf16x2_bits(O[4 * i + 2] * inv, O[4 * i + 3] * inv);
-      *reinterpret_cast<uint2*>(op + 8 * i) = w;
+      for (int b = 0; b < NB; b += 4)
+        *reinterpret_cast<f32x4*>(&o_lds[part][col][NB * (4 * grp + r) + b]) =
+            f32x4{o[0][b][r], o[0][b + 1][r], o[0][b + 2][r], o[0][b + 3][r]};
+    if (grp == 0) {
+      m_lds[part][col] = mrun;
+      l_lds[part][col] = lrun;
     }
-  } else if (kbeg < lim) {
-    const int64_t pidx = oh * max_splits + split;
-    float* op = part_o + pidx * DH + 32 * db + 4 * hf;
+  }
+  __syncthreads();
+
+  // merge and finish as attn_split_kernel, NB columns of one pair per thread
+  static_assert(16 * kRowsCols == 64 * NW, "16 threads per pair");
+  const int m = threadIdx.x >> 4;
+  const int d = (threadIdx.x & 15) * NB;
+  if (m >= nr * G) return;
+  const int i = r0 + m / G;
+  const int64_t oh = (int64_t)i * H + g * G + m % G;
+  const int len = kv_len[i];
+  float O[NB];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      *reinterpret_cast<f32x4*>(op + 8 * i) = f32x4{O[4 * i], O[4 * i + 1], O[4 * i + 2], O[4 * i + 3]};
-    if (db == 0 && hf == 0) {
+  for (int e = 0; e < NB; ++e) O[e] = 0.f;
+  auto store = [&](const float (&v)[NB]) {
+    uint32_t w[PW];
+#pragma unroll
+    for (int e = 0; e < PW; ++e) w[e] = f32x2_to_bf16x2_bits(v[2 * e], v[2 * e + 1]);
+    if constexpr (PW == 4)
+      *reinterpret_cast<u32x4*>(out + oh * DH + d) = u32x4{w[0], w[1], w[2], w[3]};
+    else
+      *reinterpret_cast<uint2*>(out + oh * DH + d) = uint2{w[0], w[1]};
+  };
+  if (len <= 0) {  // no keys: a zero row, written once
+    if (split == 0) store(O);
+    return;
+  }
+  if (kbeg >= len) return;
+  const int ns = min((len + kAttnSplit - 1) / kAttnSplit, max_splits);
+  float M = -INFINITY;
+#pragma unroll
+  for (int w = 0; w < NP; ++w) M = fmaxf(M, m_lds[w][m]);
+  float L = 0.f;
+#pragma unroll
+  for (int w = 0; w < NP; ++w) {
+    const float mw = m_lds[w][m];
+    const float f = (mw == -INFINITY) ? 0.f : exp2f(mw - M);
+#pragma unroll
+    for (int e = 0; e < NB; e += 4) {
+      const f32x4 ow = *reinterpret_cast<const f32x4*>(&o_lds[w][m][d + e]);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) O[e + c] = fmaf(ow[c], f, O[e + c]);
+    }
+    L = fmaf(l_lds[w][m], f, L);
+  }
+  if (ns == 1) {
+    const float f = (M == -INFINITY) ? 0.f : exp2f(M - M);
+#pragma unroll
+    for (int e = 0; e < NB; ++e) O[e] = attn_finish(fmaf(O[e], f, 0.f), fmaf(L, f, 0.f));
+    store(O);
+  } else {
+    const int64_t pidx = oh * max_splits + split;
+#pragma unroll
+    for (int e = 0; e < NB; e += 4)
+      *reinterpret_cast<f32x4*>(part_o + pidx * DH + d + e) = f32x4{O[e], O[e + 1], O[e + 2], O[e + 3]};
+    if (d == 0) {
       part_ml[pidx * 2] = M;
       part_ml[pidx * 2 + 1] = L;
     }
