@@ -1452,23 +1452,28 @@ static WidePlan wide_plan(int n, int tiles, int R, bool swiglu) {
   return w;
 }
 
-// Workgroup shape of the block kernel for a launch, or none. Times of one round
-// of workgroups at K = 2048 (us): 128 x 128 (16 waves) 18.5, 128 x 64 13.5 -- one per
+// Whether a one-launch many-row bf16 linear runs as the block kernel. With at
+// most kStreamMaxTiles tiles the stream kernel's one- and two-tile workgroups fill
+// more CUs up to 256 rows, below 160 of the 64 x 64 workgroups or below their 4
+// tiles (2048 x 5632 at 64 / 192 / 512 rows: stream 18 / 24 / 46, block 30 / 30 /
+// 31 us); at 32 rows or fewer and up to 512 tiles the tile kernel streams the weights
+// without barriers (q|k|v 11.7 against 12.4 us; gate|up and lm_head are faster here:
+// 16.5 -> 14.7, 30.5 -> 25.3 us).
+static bool block_takes(int n, int tiles) {
+  const long rb64 = (n + 63) / 64, g4 = (tiles + 3) / 4;
+  if (tiles <= kStreamMaxTiles) return n > 256 && tiles >= 4 && rb64 * g4 >= 160;
+  return tiles > kGemmMinBlockTiles || n > 32;
+}
+
+// Workgroup shape of the block kernel for a launch of S slices (1: the whole of K). Times of one
+// round of workgroups at K = 2048 (us): 128 x 128 (16 waves) 18.5, 128 x 64 13.5 -- one per
 // CU by their LDS -- and 64 x 64, two per CU, 11.5 for up to 256 workgroups and
 // 17 for up to 512; the shape with the fewest rounds by that measure was the
-// fastest, or within 3 %, at 64-1500 rows x 128-2000 tiles. With at most
-// kStreamMaxTiles tiles the stream kernel's one- and two-tile workgroups fill
-// more CUs up to 256 rows, below 160 of the 64 x 64 workgroups or below their 4
-// tiles (2048 x 5632 at 64 / 192 / 512 rows: stream 18 / 24 / 46,
-// block 30 / 30 / 31 us); at 32 rows or fewer and up to 512 tiles the tile kernel
-// streams the weights without barriers (q|k|v 11.7 against 12.4 us; gate|up and
-// lm_head are faster here: 16.5 -> 14.7, 30.5 -> 25.3 us).
-enum BlockShape : int { kBlockNone = 0, kBlock128x128, kBlock128x64, kBlock64x64 };
+// fastest, or within 3 %, at 64-1500 rows x 128-2000 tiles.
+enum BlockShape : int { kBlock128x128, kBlock128x64, kBlock64x64 };
 
-static int block_shape(int n, int tiles, int S) {
+static BlockShape block_shape(int n, int tiles, int S) {
   const long rb128 = (n + 127) / 128, rb64 = (n + 63) / 64, g8 = (tiles + 7) / 8, g4 = (tiles + 3) / 4;
-  if (S == 1 && ((tiles <= kStreamMaxTiles && (n <= 256 || tiles < 4 || rb64 * g4 < 160)) || (tiles <= kGemmMinBlockTiles && n <= 32)))
-    return kBlockNone;
   const long a = 37 * ((rb128 * g8 * S + 255) / 256);
   const long b = 27 * ((rb128 * g4 * S + 255) / 256);
   const long c = rb64 * g4 * S <= 256 ? 23 : 34 * ((rb64 * g4 * S + 511) / 512);
@@ -1476,7 +1481,7 @@ static int block_shape(int n, int tiles, int S) {
 }
 
 template <typename TO, int EPI, bool PART>
-static void launch_block(int shape, const void* x, const int32_t* xr, int64_t ldx, const void* W, void* y, int64_t ldy,
+static void launch_block(BlockShape shape, const void* x, const int32_t* xr, int64_t ldx, const void* W, void* y, int64_t ldy,
                          int n, int K, int tiles, bool one, int S, const RopeArgs& ra,
                          float* part, const float* rsc, hipStream_t st) {
 #define WFD_BLOCK(NW, RW, CT, ONE)                                                                              \
@@ -1531,9 +1536,9 @@ static void launch_linear(const void* x, const int32_t* xr, int64_t ldx, const v
     const float* rsc = rs.scale;  // many rows: the scales precomputed (group sums are few-row only)
     const int rb = (n + 63) / 64;
     if constexpr (std::is_same<T, bf16_t>::value) {
-      const int bs = block_shape(n, tiles, 1);
-      if (bs != kBlockNone) {
-        launch_block<TO, EPI, false>(bs, x, xr, ldx, W, y, ldy, n, K, tiles, R == 1, 1, ra, nullptr, rsc, st);
+      if (block_takes(n, tiles)) {
+        launch_block<TO, EPI, false>(block_shape(n, tiles, 1), x, xr, ldx, W, y, ldy, n, K, tiles, R == 1, 1, ra,
+                                     nullptr, rsc, st);
         return;
       }
     }
@@ -1551,8 +1556,8 @@ static void launch_linear(const void* x, const int32_t* xr, int64_t ldx, const v
                            (const T*)x, xr, ldx, (const T*)W, (TO*)y, ldy, n, K, pair_off, tiles, ra, rsc);
       return;
     }
-    // few (row block, tile) pairs (bf16: at most 32 rows): every wave streams its
-    // own weights, no barriers
+    // few (row block, tile) pairs (bf16: at most 32 rows): every wave
+    // streams its own weights, no barriers
     if (std::is_same<T, bf16_t>::value || rb * tiles <= kGemmMinBlockTiles || (n <= 32 && (tiles + 3) / 4 < 256)) {
       constexpr int NB = 2;
       hipLaunchKernelGGL((linear_tile_kernel<T, TO, EPI, NB>), dim3(rb, (tiles + NB - 1) / NB), dim3(256), 0, st,
