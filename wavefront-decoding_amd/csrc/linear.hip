@@ -42,7 +42,7 @@
 //  * stream (n > 16, at most 256 tiles): 64 rows x 1 or 2 tiles per
 //    workgroup, weights and x moved global -> LDS by direct-to-LDS loads
 //    through a 4-stage ring (3 chunks in flight without registers).
-//  * block (bf16; n > 16 with more than 512 tiles, n > 32 with more than 256,
+//  * block (bf16; n > 16 with more than 512 tiles, n > 64 with more than 256,
 //    else n > 256 and work enough): 64 or 128 rows x 64 or 128 columns per workgroup, half-chunk
 //    stages through an LDS ring.
 //  * gemm and block, slice forms (wfd_linear_partials): one slice of K per
@@ -1158,10 +1158,12 @@ __global__ __launch_bounds__(256) void linear_stream_kernel(const T* __restrict_
 // without MFMAs the launch takes 44 us, without loads 50, all of it 53; with 16
 // waves of half the columns each (four per SIMD to run through the others'
 // waits, a register set of 128) 49 us. Row by row, us before (stream / gemm
-// kernel) and now: gate|up + SwiGLU (11264 x 2048) at 64 / 112 / 192 / 512 / 1500 rows
-// 18 / 23 / 30 / 52 / 146 -> 14 / 18 / 24 / 44 / 109; q|k|v (6144 x 2048) 13.5 / 15 /
-// 21 / 29 / 77 -> 12 / 13 / 15 / 22 / 59; 2048 x 5632 at 512 / 1500 rows 46 / 128 ->
-// 31 / 49; lm_head (32000 x 2048) at 64 / 112 / 512 rows 32 / 43 / 127 -> 28 / 34 / 91.
+// kernel) and now, weights in the last-level cache: gate|up + SwiGLU (11264 x 2048) at
+// 64 / 112 / 192 / 512 / 1500 rows 18 / 23 / 30 / 52 / 146 -> 14 / 18 / 24 / 44 / 109 (from HBM
+// at 64 / 128 rows 16.0 / 19.2 now); q|k|v (6144 x 2048) at 112 / 192 / 512 / 1500 rows 15 /
+// 21 / 29 / 77 -> 13 / 15 / 22 / 59 (from HBM at 96 / 128 rows 14.8 / 15.1); 2048 x 5632 at 512 /
+// 1500 rows 46 / 128 -> 31 / 49; lm_head (32000 x 2048) at 64 / 112 / 512 rows 32 / 43 / 127 ->
+// 28 / 34 / 91.
 //
 // The product is formed transposed (weights as the A operand, x as B: the same
 // dot products, so the same bits): a lane ends with 4 consecutive columns of
@@ -1456,13 +1458,17 @@ static WidePlan wide_plan(int n, int tiles, int R, bool swiglu) {
 // most kStreamMaxTiles tiles the stream kernel's one- and two-tile workgroups fill
 // more CUs up to 256 rows, below 160 of the 64 x 64 workgroups or below their 4
 // tiles (2048 x 5632 at 64 / 192 / 512 rows: stream 18 / 24 / 46, block 30 / 30 /
-// 31 us); at 32 rows or fewer and up to 512 tiles the tile kernel streams the weights
-// without barriers (q|k|v 11.7 against 12.4 us; gate|up and lm_head are faster here:
-// 16.5 -> 14.7, 30.5 -> 25.3 us).
+// 31 us). At 64 rows or fewer (one row block) and up to 512 tiles the tile kernel
+// streams the weights without barriers, in twice as many workgroups; weights from
+// HBM, K = 2048, at 33 / 48 / 64 rows: 384 tiles 12.1 / 12.2 / 13.3 against 13.7 / 13.9
+// / 14.2 us, with the RoPE epilogue 13.8 / 14.1 / 14.9 against 14.5 / 14.9 / 15.3, 512
+// tiles x 4096 21.5 / 21.8 / 23.4 against 25.7 / 25.9 / 26.1; at 72 rows it reads them
+// twice (384 tiles 18.4 against 13.9), and above 512 tiles the block kernel is ahead
+// from 33 rows (560 tiles 14.7 against 18.5; lm_head at 24 rows 24.7 against 33.7).
 static bool block_takes(int n, int tiles) {
   const long rb64 = (n + 63) / 64, g4 = (tiles + 3) / 4;
   if (tiles <= kStreamMaxTiles) return n > 256 && tiles >= 4 && rb64 * g4 >= 160;
-  return tiles > kGemmMinBlockTiles || n > 32;
+  return tiles > kGemmMinBlockTiles || n > 64;
 }
 
 // Workgroup shape of the block kernel for a launch of S slices (1: the whole of K). Times of one
@@ -1556,7 +1562,7 @@ static void launch_linear(const void* x, const int32_t* xr, int64_t ldx, const v
                            (const T*)x, xr, ldx, (const T*)W, (TO*)y, ldy, n, K, pair_off, tiles, ra, rsc);
       return;
     }
-    // few (row block, tile) pairs (bf16: at most 32 rows): every wave
+    // few (row block, tile) pairs (bf16: at most 64 rows x 512 tiles): every wave
     // streams its own weights, no barriers
     if (std::is_same<T, bf16_t>::value || rb * tiles <= kGemmMinBlockTiles || (n <= 32 && (tiles + 3) / 4 < 256)) {
       constexpr int NB = 2;
