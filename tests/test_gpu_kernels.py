@@ -271,15 +271,16 @@ def test_linear_row_invariant(gpu, dtype, N):
 
 
 @pytest.mark.parametrize("K", [128, 384, 2048, 2176, 5632])
-@pytest.mark.parametrize("N", [528, 4112])
+@pytest.mark.parametrize("N", [2032, 4112, 8208])
 def test_linear_block_kernel_same_bits(gpu, N, K):
     """The block kernel's three workgroup shapes at the edges of their rows (32
     and 64 and 128 row groups with a row too many or too few), a ragged last
-    tile group (33 and 257 tiles), one and several chunks per sub-slice, fewer
+    tile group (127, 257 and 513 tiles), one and several chunks per sub-slice, fewer
     half chunks than ring stages, odd chunk counts: every row has the few-row
     kernel's bits, for bf16 and fp32 outputs, SwiGLU, row scales, gathered
     rows, pitched x, and outputs whose row pitch does not keep 4-element
-    alignment (33 tiles are the stream kernel's up to 256 rows)."""
+    alignment (127 tiles are the stream kernel's up to 256 rows, 257 the tile
+    kernel's up to 64)."""
     g = torch.Generator().manual_seed(N + K)
     n = 641
     X = torch.randn(n, K + 32, generator=g).to(torch.bfloat16).to(gpu)[:, :K]
@@ -338,12 +339,13 @@ def test_linear_block_kernel_rope_append(gpu, H, Hkv, Dh, blocks):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("N,K", [(2048, 2048), (2048, 5632), (2048, 4096), (256, 1024), (512, 384), (128, 128)])
+@pytest.mark.parametrize("N,K", [(2048, 2048), (2048, 5632), (2048, 4096), (256, 1024), (512, 384), (128, 128),
+                                 (2032, 2048), (656, 5632), (336, 128)])
 def test_linear_split_k_same_bits(gpu, dtype, N, K):
     """Split-K projections: the slice sums of linear_partials, added in slice
     order in fp32 and rounded, equal the one-launch linear bit for bit (1 to 4
-    slices: K = 128 .. 5632; 2 and 4 tiles per workgroup; row blocks with 1 to
-    64 rows), over contiguous and gathered rows; the norm that
+    slices: K = 128 .. 5632; 2 and 4 tiles per workgroup, ragged last groups of
+    127, 41 and 21 tiles; row blocks with 1 to 64 rows), over contiguous and gathered rows; the norm that
     reduces them (add_rmsnorm_split) equals linear + add_rmsnorm, including
     the kept linear rows (a_out), and matches the oracle."""
     if K % ops.linear_k_multiple(dtype):
