@@ -419,9 +419,12 @@ constexpr int group_max_rows(int G) { return G >= kAttnGroupRows ? 1 : kAttnGrou
 // Measured on the 2048-d model's layer tick (8 rows, 512-778 keys): 15.2 ->
 // 13.7 us; 2 rows 12.3 -> 10.7 us; 4 and 8 parts are slower (21 / 35 us),
 // since the repeated K reads reach HBM again whatever the dispatch order.
-// Four query heads per kv head leave one workgroup per CU (86 KB of LDS, two
-// below that), where more than 256 parts run a second round: 192 workgroups of
-// 16 segments x 3 rows x 1000 keys took 37 us in two parts each, 22 us whole.
+// Four query heads per kv head leave one workgroup per CU (138-214 registers a
+// lane; bf16 with one or two heads: 108-128, two workgroups), where more than 256
+// parts run a second round. us whole against split in two, 132 / 192 / 252 workgroups x 1000
+// keys: bf16, Dh 128 20 / 23 / 27 against 38 / 37 / 42, Dh 64 14 / 16 / 18 against 28 / 27 / 31; fp32,
+// Dh 128 37 / 38 / 45 against 64 / 64 / 70, Dh 64 19 / 23 / 28 against 36 / 35 / 43. Grouped rows (counted
+// here one by one) take as long either way, within 4 % below 240 rows x kv heads.
 // Every column keeps the unsplit arithmetic, so the split changes no bits.
 constexpr int kAttnFillWorkgroups = 256;
 constexpr int kAttnMaxVSplit = 2;
