@@ -210,6 +210,13 @@ def _bucket(n: int) -> int:
 _PACKED_PROMPT_ROWS = {"Wqkv": 640, "proj": 640, "fc": 256, "mlp_proj": 128, "adapter": 256}
 
 
+# Prompt rows up to which a packed d_model-output projection runs split-K: above,
+# the one-launch linear and a norm over its bf16 rows cost less than slices and a norm
+# over four fp32 ones (proj + norm at 96 / 128 / 160 / 192 / 256 / 384 rows: 13.8 / 14.0 / 16.2 /
+# 16.4 / 16.6 / 18.2 us in one launch, 13.0 / 13.6 / 14.9 / 15.7 / 16.9 / 21.0 split)
+_SPLIT_PROMPT_ROWS = 192
+
+
 class LoopedModel:
     """Device-resident looped LM running unions of rows through libwfd."""
 
@@ -421,16 +428,14 @@ class LoopedModel:
 
     def _linear_norm(self, xin: torch.Tensor, Wp, n: int, sc, tmp: str, w1: torch.Tensor, *, x_rows=None,
                      keep=None, **norm) -> None:
-        """norm(linear(xin) [+ res]) for a d_model-output projection: split-K
-        (slice sums, reduced inside the norm) for n in split_rows, else the
-        linear into sc[tmp] then the norm -- the same bits either way. `keep`
-        also receives the linear's output rows (the adapter's, which are the
-        core block's residual)."""
+        """norm(linear(xin) [+ res]) for a d_model-output projection of the prompt
+        pass: split-K (slice sums, reduced inside the norm) for n in split_rows
+        up to _SPLIT_PROMPT_ROWS, else the linear into sc[tmp] then the norm --
+        the same bits either way. `keep` also receives the linear's output rows
+        (the adapter's, which are the core block's residual)."""
         lo, hi = self.split_rows
         eps = self.cfg.norm_eps
-        # above 128 rows the one-launch linear (proj 11-13 us) and a norm over its
-        # bf16 rows cost less than slices (12-14 us) and a norm over four fp32 ones
-        if lo <= n <= min(hi, 128):
+        if lo <= n <= min(hi, _SPLIT_PROMPT_ROWS):
             S = ops.linear_partials(xin, Wp, sc["part"], n=n, x_rows=x_rows)
             ops.add_rmsnorm_split(sc["part"], S, n, w1, eps, dtype=self.dtype, a_out=keep, **norm)
         else:
