@@ -23,6 +23,7 @@ from tests.conftest import rel_err
 from wavefront_decoding_amd import model as M
 from wavefront_decoding_amd.blocks import LoopedBlocks, LoopedBlocksBatch
 from wavefront_decoding_amd.emu import EmulatedAcceptance
+from wavefront_decoding_amd import engine
 from wavefront_decoding_amd.engine import LoopedModel
 from wavefront_decoding_amd.policy import SsdPolicy
 from wavefront_decoding_amd.scheduler import generate_wavefront_dynamic
@@ -104,13 +105,17 @@ def test_prompt_pass_library_gemm_matches_kernels(gpu, dtype):
 
 
 @pytest.mark.parametrize("L", [128, 129, 257, 641])
-def test_prompt_pass_mixes_packed_and_library_linears(gpu, L):
+def test_prompt_pass_mixes_packed_and_library_linears(gpu, monkeypatch, L):
     """bf16 prompts on both sides of the row counts up to which each linear of
     the pass stays on the packed kernels (down 128, gate|up and the adapter 256,
-    q|k|v and proj 640): the slot caches and the logits agree with the pass that
+    q|k|v and proj 640, taken here for this model's own sizes): the slot caches and the logits agree with the pass that
     never leaves them, to the tolerance of the two GEMM orders' roundings."""
     import dataclasses
     cfg = dataclasses.replace(TINY, dtype="bfloat16")
+    D, F = cfg.d_model, cfg.ffn
+    for leaf, NK in dict(Wqkv=(cfg.qkv_dim, D), proj=(D, cfg.n_heads * cfg.head_dim), fc=(2 * F, D), mlp_proj=(D, F),
+                         adapter=(D, 2 * D)).items():
+        monkeypatch.setitem(engine._PACKED_PROMPT_ROWS, leaf, (engine._PACKED_PROMPT_ROWS[leaf][0], *NK))
     w = M.init_weights(cfg, 0)
     ids = _prompt(L).tolist()
     outs = []

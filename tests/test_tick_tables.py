@@ -310,3 +310,17 @@ def test_note_writes_matches_note_write():
             a.drop_positions_at_and_after(bq, at)
             b.drop_positions_at_and_after(bq, at)
         assert a.seqlen == b.seqlen
+
+
+def test_packed_prompt_rows_follow_the_weights():
+    """The prompt pass's lines between packed and library linears hold for the
+    weights they were measured with; a weight of another size has its line at
+    the same rows x N x K."""
+    from wavefront_decoding_amd import engine
+    from wavefront_decoding_amd.model import CONFIGS
+
+    measured = {leaf: rows for leaf, (rows, _, _) in engine._PACKED_PROMPT_ROWS.items()}
+    assert engine._packed_prompt_rows(CONFIGS["looped-2048"]) == measured
+    assert engine._packed_prompt_rows(CONFIGS["looped-2048-gqa"]) == measured | {"Wqkv": 2 * measured["Wqkv"]}
+    half = CONFIGS["looped-2048"].with_(d_model=1024, n_heads=8, n_kv_heads=8, ffn=2816)
+    assert engine._packed_prompt_rows(half) == {leaf: 4 * rows for leaf, rows in measured.items()}

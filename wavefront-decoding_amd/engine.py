@@ -199,22 +199,38 @@ def _bucket(n: int) -> int:
     return b
 
 
-# Prompt rows up to which each bf16 linear of the prompt pass stays on the packed
+# (rows, N, K) up to which each bf16 linear of the prompt pass stays on the packed
 # kernels (q|k|v with its RoPE + append epilogue, gate|up with its SwiGLU) although
-# the library GEMM is at hand: us per call on the 2048-d model at 128 / 256 / 512 /
-# 640 / 768 / 1024 rows, packed against library (+ epilogue launch): q|k|v 15 / 18 /
-# 24 / 25 / 39 / 45 against 33 / 34 / 34 / 35 / 37 / 41; proj 11 / 12 / 13 / 15 / 15 / 16
-# against 19 throughout; gate|up 19 / 24 / 44 / 45 / 60 / 65 against 30 / 31 / 36 / 38 /
-# 48 / 58; down 18 / 25 / 31 / 37 against 19 / 21 / 26 / 33; adapter 14 / 19 / 23 / 28
-# against 19 / 19 / 21 / 24. Below ~20 us the library call is bound by its host side.
-_PACKED_PROMPT_ROWS = {"Wqkv": 640, "proj": 640, "fc": 256, "mlp_proj": 128, "adapter": 256}
-
+# the library GEMM is at hand, and the size of the weight the rows were measured
+# with; a weight of another size has its line at the same amount of matrix work
+# (_packed_prompt_rows). us on the GPU, weights from HBM, with the epilogue or norm launch
+# that follows, at 128 / 256 / 512 / 640 / 768 / 1024 rows, packed against library: q|k|v
+# 15 / 19 / 25 / 25 / 39 / 45 against 24 / 34 / 34 / 34 / 37 / 40; proj 14 / 17 / 19 / 22 / 22 / 23
+# against 16 / 17 / 19 / 21 / 21 / 23 (within 5 % of each other up to 1536 rows: it leaves
+# with q|k|v); gate|up 20 / 25 / 45 / 45 / 61 / 67 against 23 / 32 / 37 / 39 / 48 / 58; down (one
+# launch) 23 / 29 / 37 / 44 / 44 / 45 against 21 / 26 / 32 / 39 / 38 / 45; adapter 14 / 19 / 24 / 28 / 28
+# / 29 against 13 / 16 / 21 / 24 / 24 / 28. Of the last two the short launches stay
+# packed because the pass is bound by its host side there, and a library call
+# costs it ~19 us. A quarter of the weight (1024-d, K 1024): q|k|v ahead to 1536 rows, gate|up
+# to 640 (15 against 21; 768: 26 against 23), proj to 1536; q|k|v of 16 over 4 heads ahead to 1024
+# (24 against 30), behind at 1536 (43 against 34).
+_PACKED_PROMPT_ROWS = {"Wqkv": (640, 6144, 2048), "proj": (640, 2048, 2048), "fc": (256, 11264, 2048),
+                       "mlp_proj": (128, 2048, 5632), "adapter": (256, 2048, 4096)}
 
 # Prompt rows up to which a packed d_model-output projection runs split-K: above,
 # the one-launch linear and a norm over its bf16 rows cost less than slices and a norm
 # over four fp32 ones (proj + norm at 96 / 128 / 160 / 192 / 256 / 384 rows: 13.8 / 14.0 / 16.2 /
 # 16.4 / 16.6 / 18.2 us in one launch, 13.0 / 13.6 / 14.9 / 15.7 / 16.9 / 21.0 split)
 _SPLIT_PROMPT_ROWS = 192
+
+
+def _packed_prompt_rows(cfg: LoopedLMConfig) -> dict[str, int]:
+    """Prompt rows up to which each linear of this model stays on the packed kernels."""
+    D = cfg.d_model
+    shapes = {"Wqkv": (cfg.qkv_dim, D), "proj": (D, cfg.n_heads * cfg.head_dim), "fc": (2 * cfg.ffn, D),
+              "mlp_proj": (D, cfg.ffn), "adapter": (D, 2 * D)}
+    return {leaf: rows * N * K // (shapes[leaf][0] * shapes[leaf][1])
+            for leaf, (rows, N, K) in _PACKED_PROMPT_ROWS.items()}
 
 
 class LoopedModel:
@@ -423,7 +439,7 @@ class LoopedModel:
     def _library_linears(self, n: int) -> frozenset:
         """The linears that a prompt pass over n rows runs as library GEMMs: with
         dense_prompt, those beyond the packed kernels' range (bf16), or all (fp32)."""
-        return frozenset(leaf for leaf, rows in _PACKED_PROMPT_ROWS.items()
+        return frozenset(leaf for leaf, rows in _packed_prompt_rows(self.cfg).items()
                          if self.dense_prompt and (self.dtype != torch.bfloat16 or n > rows))
 
     def _linear_norm(self, xin: torch.Tensor, Wp, n: int, sc, tmp: str, w1: torch.Tensor, *, x_rows=None,
