@@ -41,11 +41,11 @@ enum { WFD_EPI_PLAIN = 0, WFD_EPI_SWIGLU = 1 };
 
 /* Message for the last failing call on this thread. */
 const char* wfd_last_error(void);
-/* Bumped whenever an entry point's signature changes (5: wfd_argmax's
+/* Bumped whenever an entry point's signature changes or one is added (5: wfd_argmax's
    accept flags, wfd_attn_varlen_rows; 6: wfd_linear_argmax, wfd_argmax_groups;
    7: folded norm pairs -- wfd_linear_prep, wfd_norm_prep, the row-scale argument of
-   wfd_linear, wfd_linear_qkv_rope_append and wfd_linear_argmax; wfd_attn_varlen
-   joined at 7, which changed no signature). */
+   wfd_linear, wfd_linear_qkv_rope_append and wfd_linear_argmax; 8: wfd_attn_varlen,
+   which some libraries that answer 7 have too). */
 int wfd_abi_version(void);
 
 /*

@@ -35,7 +35,7 @@ def test_library_loads_and_exports_every_symbol():
 
 def test_host_only_entry_points():
     lib = _lib.load()
-    assert lib.wfd_abi_version() == 7
+    assert lib.wfd_abi_version() == 8
     # column groups of the tile argmax: 2000 tiles at <= 16 rows (lm_head), half tiles below 256 tiles,
     # none at 17 rows, for fp32 or for a K the few-row kernel does not take
     assert lib.wfd_linear_argmax_groups(8, 32000, 2048, _lib.BF16) == 2000
