@@ -324,3 +324,45 @@ def test_packed_prompt_rows_follow_the_weights():
     assert engine._packed_prompt_rows(CONFIGS["looped-2048-gqa"]) == measured | {"Wqkv": 2 * measured["Wqkv"]}
     half = CONFIGS["looped-2048"].with_(d_model=1024, n_heads=8, n_kv_heads=8, ffn=2816)
     assert engine._packed_prompt_rows(half) == {leaf: 4 * rows for leaf, rows in measured.items()}
+
+
+@pytest.mark.parametrize("name", ["LoopedModel", "_Captured"])
+def test_release_waits_for_a_capture(name):
+    """An engine (or a graph of one) whose last reference another thread drops
+    while a capture runs gives up what it holds after the capture, not inside
+    it; one dropped outside a capture does so at once."""
+    import threading
+
+    from wavefront_decoding_amd import engine
+
+    class Held:  # stands for the graph, pinned buffer or event of an engine
+        def __init__(self):
+            self.gone = threading.Event()
+
+        def __del__(self):
+            self.gone.set()
+
+    cls = getattr(engine, name)
+
+    def owner():
+        o, held = cls.__new__(cls), Held()
+        o.held = held
+        return [o], held.gone
+
+    refs, gone = owner()
+    refs.clear()
+    assert gone.is_set()
+    refs, gone = owner()
+    started = threading.Event()
+
+    def drop():
+        started.set()
+        refs.clear()
+
+    t = threading.Thread(target=drop)
+    with engine._no_release():
+        t.start()
+        assert started.wait(10)
+        assert not gone.wait(0.3)
+    assert gone.wait(10)
+    t.join(10)

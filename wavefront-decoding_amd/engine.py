@@ -88,19 +88,20 @@ class _Staging:
         return out
 
 
-_no_gc_lock = threading.RLock()
+_capture_lock = threading.RLock()  # held while this module captures, and while it releases an engine
 
 
 @contextlib.contextmanager
-def _no_gc():
-    """Python's cyclic collector held off while a stream is being captured. An
-    engine that sits in a reference cycle is freed by whichever allocation
-    happens to trigger a collection; inside a capture its destructors would
-    synchronize, destroy graphs and events and return pinned buffers whose
-    stream use the allocator records -- calls a capturing process may not
-    make, and an error raised in a destructor ends the process. Captures of
-    several threads take turns."""
-    with _no_gc_lock:
+def _no_release():
+    """Engines are not released while a stream is being captured. Their
+    destructors synchronize, destroy graphs and events and return pinned buffers
+    whose stream use the allocator records -- calls a capturing process may not
+    make, and an error raised in a destructor ends the process. An engine that
+    sits in a reference cycle is freed by whichever allocation happens to trigger
+    a collection: the cyclic collector is held off. One whose last reference
+    another thread drops waits for the capture to end (_Captured.__del__,
+    LoopedModel.__del__). Captures of several threads take turns."""
+    with _capture_lock:
         was = gc.isenabled()
         gc.disable()
         try:
@@ -149,12 +150,14 @@ class _Captured:
         self.tick.launch(self.exec if replay else 0, stream, self.events[j], self.host_ptr[j], self.dev.data_ptr(),
                          t64, self.n64, t32, self.n32, flags[0], flags[1])
 
-    def __del__(self):
-        for e in getattr(self, "events", ()):
-            try:
-                self.tick.event_destroy(e)
-            except Exception:  # interpreter shutdown: the runtime may be gone
-                pass
+    def __del__(self, lock=_capture_lock):
+        with lock:
+            for e in getattr(self, "events", ()):
+                try:
+                    self.tick.event_destroy(e)
+                except Exception:  # interpreter shutdown: the runtime may be gone
+                    pass
+            self.__dict__.clear()  # the graph and the pinned buffers, here and not after the lock
 
 
 # weights read by the linear kernels (the rest -- embedding, norms -- stay plain)
@@ -643,7 +646,7 @@ class LoopedModel:
         self._launch_plans(cache, plans, g.d32, g.d64, cache.S)                   # warm-up, then capture
         torch.cuda.synchronize()
         g.graph = torch.cuda.CUDAGraph()
-        with _no_gc(), torch.cuda.graph(g.graph):
+        with _no_release(), torch.cuda.graph(g.graph):
             self._launch_plans(cache, plans, g.d32, g.d64, cache.S)
         torch.cuda.synchronize()
         g.exec = g.graph.raw_cuda_graph_exec()
@@ -787,15 +790,16 @@ class LoopedModel:
         self._accept_unread = self._flags_pending = False
         return flags[: self._accept_n]
 
-    def __del__(self):
-        host = getattr(self, "_flags_host", 0)
-        if host:
-            try:  # no kernel may still write the flags when they are freed
-                torch.cuda.synchronize(self.device)
-                self._tick.host_free(host)
-            except Exception:  # interpreter shutdown: the runtime may be gone
-                pass
-            self._flags_host = 0
+    def __del__(self, lock=_capture_lock):
+        with lock:
+            host = getattr(self, "_flags_host", 0)
+            if host:
+                try:  # no kernel may still write the flags when they are freed
+                    torch.cuda.synchronize(self.device)
+                    self._tick.host_free(host)
+                except Exception:  # interpreter shutdown: the runtime may be gone
+                    pass
+            self.__dict__.clear()  # graphs, pinned buffers and events, here and not after the lock
 
     def prelude_union(self, cache, seqs, positions, token_ids) -> np.ndarray:
         """Embed + prelude blocks for n new tokens; fills pool[row] = [s0(pos) | e].
