@@ -140,8 +140,10 @@ def test_tables_of_two_threads_on_one_stream(monkeypatch):
 
 
 def test_split_workspace_belongs_to_its_stream(monkeypatch):
-    """The workspace attn_decode takes when none is passed: one per stream,
-    replaced only when a launch needs more; a capturing stream's is its own."""
+    """The workspace attn_decode takes when none is passed: one per stream and
+    thread, replaced only when a launch needs more; a capturing stream's is its own."""
+    import threading
+
     stream, capturing = [7], [False]
     monkeypatch.setattr(ops, "_raw_stream", lambda device: stream[0])
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing[0])
@@ -149,6 +151,11 @@ def test_split_workspace_belongs_to_its_stream(monkeypatch):
     ws = lambda n: ops.attn_workspace(n, 16, 128, 4096, "cpu")  # noqa: E731
     a = ws(8)
     assert a.numel() >= ops.attn_workspace_bytes(8, 16, 128, 4096) and ws(4) is a
+    other = []
+    t = threading.Thread(target=lambda: other.append(ws(8)))
+    t.start()
+    t.join(30)
+    assert other[0] is not a and ws(8) is a
     stream[0] = 8
     b = ws(8)
     assert b is not a and ws(8) is b

@@ -16,6 +16,7 @@ from __future__ import annotations
 
 import ctypes
 import math
+import threading
 from collections import OrderedDict
 
 import torch
@@ -120,7 +121,7 @@ def _prep_args(n: int, D: int, dtype, *, r_in=None, s_in=None, w_in=None, r_out=
 # ---------------------------------------------------------------------------
 # attention
 # ---------------------------------------------------------------------------
-_WS: OrderedDict[tuple, torch.Tensor] = OrderedDict()  # (device, stream) -> workspace
+_WS: OrderedDict[tuple, torch.Tensor] = OrderedDict()  # (device, stream, thread) -> workspace
 _MAX_WORKSPACES = 32
 
 
@@ -135,13 +136,15 @@ def _raw_stream(device: torch.device) -> int:
 
 def attn_workspace(n: int, H: int, Dh: int, kv_len_max: int, device) -> torch.Tensor:
     """A uint8 workspace large enough for this launch shape: the current
-    stream's, kept and grown, so that launches in flight on two streams never
-    share one. A stream under capture gets a fresh one, which the graph owns."""
+    stream's and thread's, kept and grown, so that neither launches in flight on
+    two streams nor the two kernels of a split launch, between which another
+    thread may enqueue its own on the same stream, ever share one. A stream
+    under capture gets a fresh one, which the graph owns."""
     need = attn_workspace_bytes(n, H, Dh, kv_len_max)
     dev = torch.device(device)
     if torch.cuda.is_current_stream_capturing():
         return torch.empty(max(need, 16), dtype=torch.uint8, device=dev)
-    key = (dev, _raw_stream(dev))
+    key = (dev, _raw_stream(dev), threading.get_ident())
     ws = _WS.get(key)
     if ws is None or ws.numel() < need:
         ws = _WS[key] = torch.empty(max(need, 1 << 20), dtype=torch.uint8, device=dev)
