@@ -53,6 +53,9 @@ def _table_calls(device):
     return {
         "rows": (lambda: A._dense_rows(2, 3, 2, True, device), (t(0, 0, 0, 2, 2, 2).long(), t(0, 1, 2, 0, 1, 2))),
         "rows, whole": (lambda: A._dense_rows(2, 1, 5, False, device), (t(0, 5).long(), t(5, 5))),
+        "one batch row": (lambda: A._dense_rows(1, 3, 5, True, device), (t(0, 0, 0).long(), t(3, 4, 5))),
+        "one batch row, whole": (lambda: A._dense_rows(1, 2, 5, False, device), (t(0, 0).long(), t(5, 5))),
+        "lone rows": (lambda: A._dense_rows(3, 1, 4, True, device), (t(0, 4, 8).long(), t(4, 4, 4))),
         "no keys": (lambda: A._dense_rows(2, 2, 0, True, device), (t(0, 0, 0, 0).long(), t(0, 0, 0, 0))),
         "prefill": (lambda: A._prefill_segments(3, 4, 7, device), (t(0, 7, 14).long(), t(0, 4, 8, 12), t(3, 3, 3))),
         "offsets": (lambda: A._dense_offsets(2, 4, 7, device), (t(0, 4, 8), t(0, 7, 14))),
@@ -71,6 +74,7 @@ def test_tables_under_capture_belong_to_the_graph(monkeypatch):
     for name, (call, want) in _table_calls(torch.device("cpu")).items():
         kept = call()
         assert all(torch.equal(a, b) and a.dtype == b.dtype for a, b in zip(kept, want, strict=True)), name
+        assert all(a.is_contiguous() for a in kept), name  # the kernels read them by their address
         assert all(a is b for a, b in zip(call(), kept)), name
         before = set(A._TABLES.held)
         for s in (7, 8):  # the warmed-up stream, and the one torch.cuda.graph captures on

@@ -237,7 +237,7 @@ def test_attn_varlen_q1_padded_matches_oracle(gpu, dtype):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("B,Tq,Tk,H,Hkv,Dh", [(2, 200, 200, 16, 4, 128), (3, 7, 150, 4, 4, 64),
-                                             (1, 1, 300, 16, 16, 128), (2, 40, 20, 4, 2, 64)])
+                                             (1, 1, 300, 16, 16, 128), (2, 40, 20, 4, 2, 64), (1, 9, 60, 4, 2, 64)])
 def test_attn_dense_matches_oracle(gpu, dtype, causal, B, Tq, Tk, H, Hkv, Dh):
     """Bottom-right causal (or full) dense attention over (B, T, H, Dh)
     batches: bf16 prompts go through the MFMA prefill kernel, the rest through

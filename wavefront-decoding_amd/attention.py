@@ -131,11 +131,11 @@ def _scale(Dh: int) -> float:
 
 def _dense_rows(B: int, Tq: int, Tk: int, causal: bool, device) -> tuple[torch.Tensor, torch.Tensor]:
     def build():
-        base = torch.arange(B, dtype=torch.int64, device=device).mul_(Tk).view(B, 1).expand(B, Tq).reshape(-1)
+        base = torch.arange(B, dtype=torch.int64, device=device).mul_(Tk).repeat_interleave(Tq)
         if not causal:
             return base, torch.full((B * Tq,), Tk, dtype=torch.int32, device=device)
         kv = torch.arange(Tk - Tq + 1, Tk + 1, dtype=torch.int32, device=device).clamp_(min=0)
-        return base, kv.expand(B, Tq).reshape(-1)
+        return base, kv.repeat(B)
 
     return _cached(device, ("dense", B, Tq, Tk, causal), build)
 
