@@ -38,7 +38,7 @@ def _p(t: torch.Tensor | None) -> int | None:
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _need_cuda(*ts: torch.Tensor | None) -> None:
@@ -141,7 +141,7 @@ def attn_workspace(n: int, H: int, Dh: int, kv_len_max: int, device) -> torch.Te
     thread may enqueue its own on the same stream, ever share one. A stream
     under capture gets a fresh one, which the graph owns."""
     need = attn_workspace_bytes(n, H, Dh, kv_len_max)
-    dev = torch.device(device)
+    dev = device if isinstance(device, torch.device) else torch.device(device)
     if torch.cuda.is_current_stream_capturing():
         return torch.empty(max(need, 16), dtype=torch.uint8, device=dev)
     key = (dev, _raw_stream(dev), threading.get_ident())
