@@ -159,10 +159,10 @@ def _shared_rows(total_q: int, nseg: int, max_k: int, H: int, Hkv: int, Dh: int)
     empty: it wins below two rows a segment and up to some rounds of its
     workgroups: three of 256 at Dh 128, one with four query heads per kv head
     (which it takes longest over), four of the half as long ones at Dh 64. us,
-    decode against this kernel, by workgroups: Dh 128, 16 heads: 384 16.1 / 24.2, 736
-    13.0 / 13.3, 1568 21 / 14 and 43 / 27, 4960 99 / 52, 32384 735 / 168; 16 heads
-    over 4: 164 10.1 / 13.4, 268 24.6 / 23.0, 392 33 / 26, 8096 460 / 122; Dh 64, 4
-    heads: 512 9.7 / 14.1, 704 24 / 31, 1480 15.6 / 11.2, 8096 111 / 45."""
+    decode against this kernel, by workgroups: Dh 128, 16 heads: 384 16.0 / 21.6, 736
+    13.0 / 13.0, 1568 21 / 13 and 43 / 27, 4960 100 / 52, 32384 726 / 164; 16 heads
+    over 4: 164 10.2 / 13.1, 268 24.5 / 21.4, 392 33 / 24, 8096 458 / 114; Dh 64, 4
+    heads: 512 9.6 / 13.6, 704 24 / 29, 1480 15.5 / 10.7, 8096 110 / 43."""
     if total_q < 2 * nseg or Dh not in (64, 128) or Hkv <= 0 or H not in (Hkv, 2 * Hkv, 4 * Hkv):
         return False
     return total_q * Hkv * ((max_k + 1023) // 1024) > (1024 if Dh == 64 else 256 if H == 4 * Hkv else 768)

@@ -31,14 +31,16 @@
 //    (attn_combine_kernel).
 //
 // What bounds it: issue. A tile of 16 pairs x 32 keys x 128 columns is 64 fp32
-// products of 32 cycles, a third of the time of 48 segments of 1-64 rows over
-// 100-2048 keys x 16 heads x 128 (394 MB of K and V): 168 us (the tables 5, this
-// kernel 152, the merge of splits 10) against 720 for the row form. The chains
-// take 128 registers, so a CU holds 8 waves: as two workgroups of 4 waves with
-// two parts each, so that one's loads and merge run under the other's products
-// (one workgroup of 8 waves: 209 us; with the merge's factors computed once per
-// output, 182). K and V of the next tile are loaded as soon as the registers of
-// this one's are free.
+// products of 32 cycles, 44 % of the time that a CU is busy with 48 segments of
+// 1-64 rows over 100-2048 keys x 16 heads x 128 (394 MB of K and V): 164 us (the
+// tables 5, this kernel 147, the merge of splits 10) against 720 for the row form;
+// a fifth of the time CUs wait for the last workgroups. The chains take 128
+// registers, so a CU holds 8 waves: as two workgroups of 4 waves with two parts each,
+// so that one's loads and merge run under the other's products (one workgroup of 8
+// waves: 209 us; with the merge's factors computed once per output 182; with one
+// conversion between two products, which costs the matrix core some ten cycles,
+// masks and denormal handling in every tile 168). K and V of the next tile are
+// loaded as soon as the registers of this one's are free.
 #include "attn_combine.h"
 
 namespace wfd {
@@ -162,6 +164,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) __attribute__((amdgpu_waves_per_eu
   if (split > 0 && kbeg >= maxlen) return;  // uniform over the workgroup
   const int nkeys = max(min(maxlen, kbeg + kAttnSplit) - kbeg, 0);  // of this split
   const int nt = (nkeys + TK - 1) / TK;
+  const int np = min(nt, NP);  // parts that hold keys
 
   // K / V of this kv head from key kbeg; the resources end at the split's last
   // key, so loads of later keys read zeros and send nothing to memory
@@ -220,7 +223,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) __attribute__((amdgpu_waves_per_eu
 #pragma unroll
   for (int x = 0; x < NS * RG; ++x) fetch_v(wave, x);
 #pragma unroll 1
-  for (int part = wave; part < NP; part += NW) {
+  for (int part = wave; part < np; part += NW) {
     float mrun = -INFINITY, lrun = 0.f;
     f32x4 o[RG][NB];  // O^T by chain: columns NB (4 grp + r) + b of pair col
 #pragma unroll
@@ -242,24 +245,46 @@ __global__ __launch_bounds__(64 * kRowsWaves) __attribute__((amdgpu_waves_per_eu
       {
 #pragma clang fp contract(off)
         float mt = -INFINITY;
+        if (t0 + TK > minlen) {  // some row's last key lies in or before this tile (uniform)
 #pragma unroll
-        for (int j = 0; j < NJ; ++j)
+          for (int j = 0; j < NJ; ++j)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const float sv = t0 + key_of(j, 4 * grp) + r < lim ? p[j][r] * scale_log2 : -INFINITY;
-            p[j][r] = sv;
-            mt = fmaxf(mt, sv);
-          }
+            for (int r = 0; r < 4; ++r) {
+              p[j][r] = t0 + key_of(j, 4 * grp) + r < lim ? p[j][r] * scale_log2 : -INFINITY;
+              mt = fmaxf(mt, p[j][r]);
+            }
+        } else {
+#pragma unroll
+          for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              p[j][r] *= scale_log2;
+              mt = fmaxf(mt, p[j][r]);
+            }
+        }
         const Pair m32 = pair32(mt);
         const Pair m16 = pair16(fmaxf(m32.a, m32.b));
         mt = fmaxf(m16.a, m16.b);
         const float mnew = fmaxf(mrun, mt);
         const float corr = (mrun == -INFINITY) ? 0.f : exp2f(mrun - mnew);
         mrun = mnew;
+        // exp2f(x) is v_exp_f32(x) from -126 up, which is what most tiles hold
+        float low = 0.f;
 #pragma unroll
         for (int j = 0; j < NJ; ++j)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) p[j][r] = (p[j][r] == -INFINITY) ? 0.f : exp2f(p[j][r] - mnew);
+          for (int r = 0; r < 4; ++r) low = fminf(low, p[j][r] - mnew);
+        if (__builtin_amdgcn_ballot_w64(low >= -126.f) == ~0ull) {
+#pragma unroll
+          for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) p[j][r] = __builtin_amdgcn_exp2f(p[j][r] - mnew);
+        } else {
+#pragma unroll
+          for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) p[j][r] = (p[j][r] == -INFINITY) ? 0.f : exp2f(p[j][r] - mnew);
+        }
         // the tile's sum, by key % 16 (c) over the tile's 16-key blocks, then the
         // butterfly over c: xor 8, 4, 2, 1
         float u[4];
@@ -322,17 +347,29 @@ __global__ __launch_bounds__(64 * kRowsWaves) __attribute__((amdgpu_waves_per_eu
           }
         }
       }
+      // eight values converted, then their products: a VALU instruction between two
+      // products costs the matrix core some ten cycles
+      constexpr int XB = 8 / NB;
 #pragma unroll
-      for (int x = 0; x < NS * RG; ++x) {
+      for (int x0 = 0; x0 < NS * RG; x0 += XB) {
+        float v[XB][NB];
 #pragma unroll
-        for (int e = 0; e < PW; ++e) {
-          f32x4& lo = o[x % RG][2 * e];
-          f32x4& hi = o[x % RG][2 * e + 1];
-          lo = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(vreg[x][e] << 16), p[x / 4][x % 4], lo, 0, 0, 0);
-          hi = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(vreg[x][e] & 0xffff0000u), p[x / 4][x % 4], hi, 0, 0,
-                                                    0);
-        }
-        fetch_v(tn, x);
+        for (int x = 0; x < XB; ++x)
+#pragma unroll
+          for (int e = 0; e < PW; ++e) {
+            v[x][2 * e] = __uint_as_float(vreg[x0 + x][e] << 16);
+            v[x][2 * e + 1] = __uint_as_float(vreg[x0 + x][e] & 0xffff0000u);
+          }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int x = x0; x < x0 + XB; ++x)
+#pragma unroll
+          for (int b = 0; b < NB; ++b)
+            o[x % RG][b] =
+                __builtin_amdgcn_mfma_f32_16x16x4f32(v[x - x0][b], p[x / 4][x % 4], o[x % RG][b], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int x = x0; x < x0 + XB; ++x) fetch_v(tn, x);
       }
     }
 
@@ -383,11 +420,9 @@ __global__ __launch_bounds__(64 * kRowsWaves) __attribute__((amdgpu_waves_per_eu
   if (kbeg >= len) return;
   const int ns = min((len + kAttnSplit - 1) / kAttnSplit, max_splits);
   float M = -INFINITY;
-#pragma unroll
-  for (int w = 0; w < NP; ++w) M = fmaxf(M, m_lds[w][m]);
+  for (int w = 0; w < np; ++w) M = fmaxf(M, m_lds[w][m]);
   float L = 0.f;
-#pragma unroll
-  for (int w = 0; w < NP; ++w) {
+  for (int w = 0; w < np; ++w) {
     const float mw = m_lds[w][m];
     const float f = (mw == -INFINITY) ? 0.f : exp2f(mw - M);
 #pragma unroll
@@ -398,6 +433,8 @@ __global__ __launch_bounds__(64 * kRowsWaves) __attribute__((amdgpu_waves_per_eu
     }
     L = fmaf(l_lds[w][m], f, L);
   }
+#pragma unroll
+  for (int e = 0; e < NB; ++e) O[e] += np < NP ? 0.f : -0.f;  // parts without keys add +0, others nothing
   if (ns == 1) {
     const float f = (M == -INFINITY) ? 0.f : exp2f(M - M);
 #pragma unroll
