@@ -334,7 +334,7 @@ int wfd_linear_slices(int K, int dtype);
 /*
  * Split-K form of wfd_linear (plain epilogue): one workgroup per (64 or 128 rows,
  * 32 to 128 columns, K slice), so a many-row projection with few output
- * columns fills the chip and reads each x row once per 32-64 columns. Writes
+ * columns fills the chip and reads each x row once per 32 to 128 columns. Writes
  * the fp32 slice sums part[(q * n + m) * N + j] for q < wfd_linear_slices(K);
  * adding them in slice order from zero and rounding to dtype gives wfd_linear's
  * y[m, j] bit for bit (wfd_add_rmsnorm_split does exactly that). Shapes,
