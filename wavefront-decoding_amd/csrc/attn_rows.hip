@@ -32,7 +32,8 @@
 //
 // What bounds it: issue. A tile of 16 pairs x 32 keys x 128 columns is 64 fp32
 // products of 32 cycles, 44 % of the time that a CU is busy with 48 segments of
-// 1-64 rows over 100-2048 keys x 16 heads x 128 (394 MB of K and V): 164 us (the
+// 1-64 rows over 100-2048 keys x 16 heads x 128 (394 MB of K and V), and vector
+// instructions another 37 %; the two do not overlap, also across waves. 164 us (the
 // tables 5, this kernel 147, the merge of splits 10) against 720 for the row form;
 // a fifth of the time CUs wait for the last workgroups. The chains take 128
 // registers, so a CU holds 8 waves: as two workgroups of 4 waves with two parts each,
